@@ -733,7 +733,18 @@ struct FwdResArgs {
     int mark;                   // failure mark in *status (forced_timeout)
     int local_ok;               // XCD-local exchange stores allowed (local_exchange_allowed)
     int lagged_shift;           // shift the row exponentials by the last iteration's LSE
+    int scaling;                // start in the scaling domain (forward)
 };
+
+// Bounds of the scaling domain (forward): the column factors V and the row
+// factors w of a workgroup's element stay within them, or the element goes
+// back to the log domain.  An entry E below 2^-126 may be flushed to 0; with
+// M <= 1024 rows its share of a column sum r = sum_i E w is at most
+// 2^10 2^-126 2^40 = 2^-76, and r >= 2^-50 keeps that below 2^-26 of r.  In a
+// row, s >= 2^-40 (the largest E is 1) against 2^10 2^-126 2^40.
+constexpr float kScaleMax = 0x1p40f;
+constexpr float kScaleMin = 0x1p-40f;
+constexpr float kScaledColMin = 0x1p-50f;
 
 // Waits for G tagged per-workgroup deltas of iteration t and returns their
 // maximum (order-free, so every workgroup gets the same value).  Every thread
@@ -789,7 +800,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     float* lds_la = lds_u + 2 * ROWS;
     float* scratch = lds_la + ROWS;  // [0] global delta, [1..kWaves] wave deltas, [16..] reductions
     const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // row addresses in scalar registers
     const int G = gridDim.x;
     const int gid = logical_group(a.W);
     const int b = gid / a.W;
@@ -803,20 +814,29 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     const float pad = a.kscale > 0.0f ? -INFINITY : INFINITY;
     announce_xcc(a.xchg, a.N, b, a.W, w, a.xcc_tag);
 
-    float x[RPW][PL];
+    float x[RPW][PL];  // the scores of this wave's rows, or E in the scaling domain
+    auto load_scores = [&]() {
+        // opaque copies: the row addresses and column masks are formed at each
+        // of the two uses instead of being kept from the first to the second
+        int r0 = row0, ln = lane;
+        asm volatile("" : "+s"(r0));
+        asm volatile("" : "+v"(ln));
 #pragma unroll
-    for (int k = 0; k < RPW; ++k) {
-        const int i = row0 + wave + kWaves * k;
-        if (i < rend) {
-            R::load(a.X + (bM + i) * a.N, lane, a.N, x[k], 0.0f);
+        for (int k = 0; k < RPW; ++k) {
+            const int i = r0 + wave + kWaves * k;
+            if (i < rend) {
+                R::load(a.X + (bM + i) * a.N, ln, a.N, x[k], 0.0f);
 #pragma unroll
-            for (int e = 0; e < PL; ++e)
-                if (!R::valid(lane, e, a.N)) x[k][e] = pad;
-        } else {
+                for (int e = 0; e < PL; ++e)
+                    if (!R::valid(ln, e, a.N)) x[k][e] = pad;
+            } else {
 #pragma unroll
-            for (int e = 0; e < PL; ++e) x[k][e] = pad;
+                for (int e = 0; e < PL; ++e) x[k][e] = pad;
+            }
         }
-    }
+    };
+    load_scores();
+    bool scal = !SCHED && a.scaling && a.max_iter > 0;
     for (int l = threadIdx.x; l < ROWS; l += kThreads) {
         const int i = row0 + l;
         lds_la[l] = (i < rend && a.log_a) ? a.log_a[bM + i] : a.log_a_default;
@@ -825,13 +845,13 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     }
     for (int j = threadIdx.x; j < a.N; j += kThreads) {
         lds_lb[j] = a.log_b ? a.log_b[bN + j] : a.log_b_default;
-        lds_v[j] = 0.0f;
-        lds_v[a.N + j] = 0.0f;
+        lds_v[j] = scal ? 1.0f : 0.0f;
+        lds_v[a.N + j] = scal ? 1.0f : 0.0f;
     }
     __syncthreads();
-    float v[PL];
+    float v[PL];  // v_{t-1}, or V_{t-1} in the scaling domain
 #pragma unroll
-    for (int e = 0; e < PL; ++e) v[e] = 0.0f;
+    for (int e = 0; e < PL; ++e) v[e] = scal ? 1.0f : 0.0f;
     // log a of the row this lane takes in each group of GR rows
     float lga_slot[RPW / GR];
 #pragma unroll
@@ -843,6 +863,45 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     // scheduled runs: this iteration's scale, and the next one's already in flight
     float ks_it = a.kscale;
     float ks_next = (SCHED && a.max_iter > 0) ? a.kscale_t[0] : a.kscale;
+    // Scaling domain: each lane keeps the values of one of its wave's rows,
+    // row slot_of_lane (four lanes share a row), and each thread b of its columns.
+    const int lslot = wave + kWaves * slot_of_lane<RPW>(lane);
+    const bool row_ok = row0 + lslot < rend;
+    const bool row_owner = lane < 16 && (lane & (16 / RPW - 1)) == 0 && row_ok;
+    float m_l = 0.0f, a_l = 0.0f, w_l = 0.0f, w_prev = 0.0f, u_prev = 0.0f;
+    float b_own[kColRounds<PL>] = {};
+    if constexpr (!SCHED) {
+        if (scal) {
+            float lm[RPW];
+#pragma unroll
+            for (int k = 0; k < RPW; ++k) {
+                lm[k] = -FLT_MAX;
+#pragma unroll
+                for (int e = 0; e < PL; ++e) lm[k] = fmaxf(lm[k], x[k][e] * kscale2);
+            }
+            m_l = transposed_reduce<RPW>(lm, OpMax{});
+            // what the rounding of kscale log2(e) left out, times a finite x (an
+            // infinite one has its infinity from the first term already)
+            constexpr float kLog2ELo = 1.92596303e-8f;  // log2 e - kLog2E
+            const float kscale2_lo = fmaf(a.kscale, kLog2ELo, fmaf(a.kscale, kLog2E, -kscale2));
+#pragma unroll
+            for (int k = 0; k < RPW; ++k) {
+                const float m = read_lane(m_l, lane_of_slot<RPW>(k));
+#pragma unroll
+                for (int e = 0; e < PL; ++e) {
+                    const float xf = fminf(fmaxf(x[k][e], -FLT_MAX), FLT_MAX);
+                    const float y = fmaf(xf, kscale2_lo, fmaf(x[k][e], kscale2, -m));
+                    x[k][e] = __builtin_amdgcn_exp2f(y);  // 0 for the padding, whose y is -inf
+                }
+            }
+            a_l = exp_compensated(lds_la[lslot]);
+#pragma unroll
+            for (int q = 0; q < kColRounds<PL>; ++q) {
+                const int j = threadIdx.x + q * kThreads;
+                if (j < a.N) b_own[q] = exp_compensated(lds_lb[j]);
+            }
+        }
+    }
     bool dead = false;
     const bool local =
         element_on_one_xcd(a.xchg, a.N, b, a.W, w, a.spin_limit, a.status, dead, scratch, a.xcc_tag, a.mark) &&
@@ -850,252 +909,343 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     int used = a.max_iter;
     int conv = 0;
 
-    for (int t = 1; t <= a.max_iter; ++t) {
-        const int cur = t & 1, prev = cur ^ 1;
-        const bool test = check && t >= 2;
-        if constexpr (SCHED) {
-            ks_it = ks_next;
-            kscale2 = ks_it * kLog2E;
-            if (t < a.max_iter) ks_next = a.kscale_t[t];
-        }
+    auto prefetch_deltas = [&](int t, unsigned long long(&dpre)[kDeltaPrefetch]) {
         unsigned long long* ds = a.dxchg + size_t((t - 1) % kDeltaSlots) * G;
-        unsigned long long dpre[kDeltaPrefetch];
-        if (test && wave == 0) {
 #pragma unroll
-            for (int q = 0; q < kDeltaPrefetch; ++q) {
-                const int g = lane + q * kWave;
-                dpre[q] = g < G ? __hip_atomic_load(ds + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                : tag_pack(0.0f, a.tag_base | unsigned(t - 1));
+        for (int q = 0; q < kDeltaPrefetch; ++q) {
+            const int g = lane + q * kWave;
+            dpre[q] = g < G ? __hip_atomic_load(ds + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                            : tag_pack(0.0f, a.tag_base | unsigned(t - 1));
+        }
+    };
+    auto publish_delta = [&](int t) {
+        float d = scratch[1];
+#pragma unroll
+        for (int q = 1; q < kWaves; ++q) d = fmaxf(d, scratch[1 + q]);
+        publish(a.dxchg + size_t(t % kDeltaSlots) * G + gid, d, a.tag_base | unsigned(t));
+    };
+    // wave 0: the batch-global change of iteration t - 1, into scratch[0]
+    auto finish_deltas = [&](int t, const unsigned long long(&dpre)[kDeltaPrefetch]) {
+        unsigned long long* ds = a.dxchg + size_t((t - 1) % kDeltaSlots) * G;
+        float gmax = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kDeltaPrefetch; ++q) {
+            const int g = lane + q * kWave;
+            if (g < G) {
+                float d = __uint_as_float(static_cast<unsigned>(dpre[q]));
+                if (static_cast<unsigned>(dpre[q] >> 32) != (a.tag_base | unsigned(t - 1)))
+                    d = collect(ds + g, a.tag_base | unsigned(t - 1), a.spin_limit, a.status, dead, a.mark);
+                gmax = OpMaxNan{}(gmax, d);
             }
         }
-        // Row update (kernels.cu:503-545) and the shared-exponential column sums,
-        // in base 2: y = K log2(e) + v log2(e), m = max_j y, s = sum_j 2^(y - m),
-        // u = log a - ln2 (m + log2 s), and the column sums take 2^(y - m) a / s.
-        // Rows go in groups of GR: their maxima and sums are reduced across the
-        // wave together (transposed butterfly), and each lane then takes the
-        // logarithm for one row of the group.
-        float acc[PL], v2[PL];
+        for (int g = lane + kDeltaPrefetch * kWave; g < G; g += kWave)
+            gmax = OpMaxNan{}(gmax, collect(ds + g, a.tag_base | unsigned(t - 1), a.spin_limit, a.status,
+                                            dead, a.mark));
+        gmax = wave_reduce(gmax, OpMaxNan{});
+        if (lane == 0) scratch[0] = gmax;
+    };
+
+    int t0 = 1;           // the log domain's first iteration
+    bool resume = false;  // ... whose row update and exchange the scaling domain has done
+    if constexpr (!SCHED) {
+        for (int t = 1; scal && t <= a.max_iter; ++t) {
+            const int cur = t & 1;
+            const bool test = check && t >= 2;
+            unsigned long long dpre[kDeltaPrefetch];
+            if (test && wave == 0) prefetch_deltas(t, dpre);
+            float acc[PL], dmax = 0.0f;
+            float d[RPW];  // one dependent chain per row; the rows give the parallelism
 #pragma unroll
-        for (int e = 0; e < PL; ++e) {
-            acc[e] = 0.0f;
-            v2[e] = v[e] * kLog2E;
+            for (int k = 0; k < RPW; ++k) {
+                d[k] = 0.0f;
+#pragma unroll
+                for (int e = 0; e < PL; ++e) d[k] = fmaf(x[k][e], v[e], d[k]);
+            }
+            const float s_sum = transposed_sum<RPW>(d);
+            const float s_l = s_sum > 0.0f ? s_sum : sk::kSumFloor;  // 0: a row with no finite K
+            w_prev = w_l;
+            w_l = a_l / s_l;
+            const float u_l = lds_la[lslot] - kLn2 * (m_l + __builtin_amdgcn_logf(s_l));
+            // a row factor out of range, or NaN: every column's sum becomes NaN,
+            // which all workgroups of the element see
+            const bool bad = __any(row_ok && s_sum != 0.0f && !(w_l <= kScaleMax));
+#pragma unroll
+            for (int e = 0; e < PL; ++e) acc[e] = bad ? __builtin_nanf("") : 0.0f;
+#pragma unroll
+            for (int k = 0; k < RPW; ++k) {
+                const float wk = read_lane(w_l, lane_of_slot<RPW>(k));
+#pragma unroll
+                for (int e = 0; e < PL; ++e) acc[e] = fmaf(x[k][e], wk, acc[e]);
+            }
+            if (check) dmax = wave_max(row_ok ? fabsf(u_l - u_prev) : 0.0f);
+            u_prev = u_l;
+            if (row_owner) {
+                lds_u[cur * ROWS + lslot] = u_l;
+                if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + row0 + lslot] = u_l;
+            }
+            // part: as in the log domain below
+            R::store(part + wave * a.N, lane, a.N, acc);
+            if (lane == 0) scratch[1 + wave] = dmax;
+            __syncthreads();
+            if (check && threadIdx.x == 0) publish_delta(t);
+            int low = 0;
+            exchange_columns<kColRounds<PL>>(
+                part, a.xchg + size_t(cur) * G * a.N, a.N, b, a.W, w, a.tag_base | unsigned(t), local,
+                a.spin_limit, a.status, dead, a.mark, [&](int j, float r) {
+                    const float vn = pick(b_own, (j - threadIdx.x) / kThreads) / r;
+                    const bool ok = r >= kScaledColMin && vn >= kScaleMin && vn <= kScaleMax;
+                    lds_v[cur * a.N + j] = ok ? vn : __builtin_nanf("");
+                    low |= !ok;
+                });
+            if (test && wave == 0) finish_deltas(t, dpre);
+            if (__syncthreads_or(low)) {  // back to the log domain, the columns marked NaN to be formed there
+                scal = false;
+                resume = true;
+                t0 = t;
+                break;
+            }
+            if (a.v_hist && w == 0)
+                for (int j = threadIdx.x; j < a.N; j += kThreads)
+                    a.v_hist[(size_t(t - 1) * a.B + b) * a.N + j] = logf(lds_v[cur * a.N + j]);
+            if (test && scratch[0] < a.tol) {  // the stop test of iteration t-1 fired
+                used = t - 1;
+                conv = 1;
+                w_l = w_prev;
+                break;
+            }
+            R::load(lds_v + cur * a.N, lane, a.N, v, 0.0f);
         }
-        float uk[RPW];  // this wave's new u values; stored after the loop, which keeps it branch-free
-#pragma unroll
-        for (int g0 = 0; g0 < RPW; g0 += GR) {
-            float y[GR][PL];
-            // The shift m of a row's exponentials: its log2-sum-exp of the
-            // previous iteration, which spares the row maximum and keeps the sum
-            // near 1 once v settles; the row maximum itself in the first
-            // iteration and whenever the shifted sum leaves [2^-30, 2^30] (a
-            // large change of v or of the scale, a row without a finite score).
-            // Within it the largest term is at least 2^-42, so every term that
-            // matters is a normal float, and the sum is above the floor
-            // (1e-12) that applies only to a maximum-shifted sum.
-            auto row_max = [&](const float (&v2)[PL]) {
-                float lm[GR];
-#pragma unroll
-                for (int r = 0; r < GR; ++r) {
-                    lm[r] = -FLT_MAX;
-#pragma unroll
-                    for (int e = 0; e < PL; ++e) lm[r] = fmaxf(lm[r], fmaf(x[g0 + r][e], kscale2, v2[e]));
-                }
-                return transposed_reduce<GR>(lm, OpMax{});
-            };
-            auto shifted_exps = [&](float m, const float (&v2)[PL]) {
-                float ls[GR];
-#pragma unroll
-                for (int r = 0; r < GR; ++r) {
-                    const float mr = read_lane(m, lane_of_slot<GR>(r));
-                    ls[r] = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < PL; ++e) {
-                        y[r][e] = __builtin_amdgcn_exp2f(fmaf(x[g0 + r][e], kscale2, v2[e]) - mr);
-                        ls[r] += y[r][e];
-                    }
-                }
-                return transposed_sum<GR>(ls);
-            };
-            const bool exact = t == 1 || !a.lagged_shift;
-            float m_l = exact ? row_max(v2) : lse_slot[g0 / GR];
-            float s_sum = shifted_exps(m_l, v2);
-            if (!exact && !__all(s_sum >= 0x1p-30f && s_sum <= 0x1p30f)) {
-                // v2 again, opaque to the compiler: kept from sharing the first
-                // pass's products, whose registers the exponentials then reuse
-                float v2r[PL];
+        if (resume) {
+            for (int j = threadIdx.x; j < a.N; j += kThreads) {  // own writes
+                lds_v[j] = logf(lds_v[j]);
+                lds_v[a.N + j] = logf(lds_v[a.N + j]);
+            }
+            load_scores();
+        }
+    }
+    if (!scal) {
+        bool first = true;  // no LSE of the last iteration to shift by
+        for (int t = t0; t <= a.max_iter && conv == 0; ++t) {
+            const int cur = t & 1, prev = cur ^ 1;
+            const bool test = check && t >= 2;
+            if constexpr (SCHED) {
+                ks_it = ks_next;
+                kscale2 = ks_it * kLog2E;
+                if (t < a.max_iter) ks_next = a.kscale_t[t];
+            }
+            unsigned long long dpre[kDeltaPrefetch];
+            if (test && wave == 0 && !resume) prefetch_deltas(t, dpre);
+            int low = resume ? 1 : 0;
+            if (!resume) {
+                // Row update (kernels.cu:503-545) and the shared-exponential column sums,
+                // in base 2: y = K log2(e) + v log2(e), m = max_j y, s = sum_j 2^(y - m),
+                // u = log a - ln2 (m + log2 s), and the column sums take 2^(y - m) a / s.
+                // Rows go in groups of GR: their maxima and sums are reduced across the
+                // wave together (transposed butterfly), and each lane then takes the
+                // logarithm for one row of the group.
+                float acc[PL], v2[PL];
 #pragma unroll
                 for (int e = 0; e < PL; ++e) {
-                    v2r[e] = v2[e];
-                    asm volatile("" : "+v"(v2r[e]));
+                    acc[e] = 0.0f;
+                    v2[e] = v[e] * kLog2E;
                 }
-                m_l = row_max(v2r);
-                s_sum = shifted_exps(m_l, v2r);
-            }
-            const float s_l = fmaxf(s_sum, sk::kSumFloor);
-            const float lga_l = lga_slot[g0 / GR];
-            const float lg2 = __builtin_amdgcn_logf(s_l);  // log2
-            const float lse = m_l + lg2;
-            lse_slot[g0 / GR] = lse;
-            const float u_l = lga_l - kLn2 * lse;
-            const float w_l = __builtin_amdgcn_exp2f(fmaf(lga_l, kLog2E, -lg2));  // a / s
+                float uk[RPW];  // this wave's new u values; stored after the loop, which keeps it branch-free
 #pragma unroll
-            for (int r = 0; r < GR; ++r) {
-                const float wr = read_lane(w_l, lane_of_slot<GR>(r));
-                uk[g0 + r] = read_lane(u_l, lane_of_slot<GR>(r));
+                for (int g0 = 0; g0 < RPW; g0 += GR) {
+                    float y[GR][PL];
+                    // The shift m of a row's exponentials: its log2-sum-exp of the
+                    // previous iteration, which spares the row maximum and keeps the sum
+                    // near 1 once v settles; the row maximum itself in the first
+                    // iteration and whenever the shifted sum leaves [2^-30, 2^30] (a
+                    // large change of v or of the scale, a row without a finite score).
+                    // Within it the largest term is at least 2^-42, so every term that
+                    // matters is a normal float, and the sum is above the floor
+                    // (1e-12) that applies only to a maximum-shifted sum.
+                    auto row_max = [&](const float (&v2)[PL]) {
+                        float lm[GR];
 #pragma unroll
-                for (int e = 0; e < PL; ++e) acc[e] = fmaf(y[r][e], wr, acc[e]);
-            }
-            // Materialise acc here: left alone, the compiler postpones the updates
-            // to the end of the loop and keeps every group's exponentials live.
+                        for (int r = 0; r < GR; ++r) {
+                            lm[r] = -FLT_MAX;
 #pragma unroll
-            for (int e = 0; e < PL; ++e) asm volatile("" : "+v"(acc[e]));
-        }
-        float dmax = 0.0f;
+                            for (int e = 0; e < PL; ++e) lm[r] = fmaxf(lm[r], fmaf(x[g0 + r][e], kscale2, v2[e]));
+                        }
+                        return transposed_reduce<GR>(lm, OpMax{});
+                    };
+                    auto shifted_exps = [&](float m, const float (&v2)[PL]) {
+                        float ls[GR];
 #pragma unroll
-        for (int k = 0; k < RPW; ++k) {
-            const int l = wave + kWaves * k;
-            const int i = row0 + l;
-            if (i < rend) {
-                dmax = fmaxf(dmax, fabsf(uk[k] - lds_u[prev * ROWS + l]));
-                if (lane == 0) {
-                    lds_u[cur * ROWS + l] = uk[k];
-                    if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + i] = uk[k];
-                }
-            }
-        }
-        // The last readers of part (the previous exchange or exact fallback)
-        // are behind the barrier that ends the previous iteration's exchange.
-        R::store(part + wave * a.N, lane, a.N, acc);
-        if (lane == 0) scratch[1 + wave] = dmax;
-        __syncthreads();
-        if (check && threadIdx.x == 0) {
-            float d = scratch[1];
+                        for (int r = 0; r < GR; ++r) {
+                            const float mr = read_lane(m, lane_of_slot<GR>(r));
+                            ls[r] = 0.0f;
 #pragma unroll
-            for (int q = 1; q < kWaves; ++q) d = fmaxf(d, scratch[1 + q]);
-            publish(a.dxchg + size_t(t % kDeltaSlots) * G + gid, d, a.tag_base | unsigned(t));
-        }
-        int low = 0;
-        exchange_columns<kColRounds<PL>>(
-            part, a.xchg + size_t(cur) * G * a.N, a.N, b, a.W, w, a.tag_base | unsigned(t), local, a.spin_limit,
-            a.status, dead, a.mark,
-            [&](int j, float cs) {
-                if (cs >= sk::kColSumFloor && cs <= FLT_MAX) {
-                    lds_v[cur * a.N + j] = lds_lb[j] + lds_v[prev * a.N + j] - logf(cs);
-                } else {
-                    lds_v[cur * a.N + j] = __builtin_nanf("");  // exact LSE below
-                    low = 1;
-                }
-            });
-        if (test && wave == 0) {
-            float gmax = 0.0f;
+                            for (int e = 0; e < PL; ++e) {
+                                y[r][e] = __builtin_amdgcn_exp2f(fmaf(x[g0 + r][e], kscale2, v2[e]) - mr);
+                                ls[r] += y[r][e];
+                            }
+                        }
+                        return transposed_sum<GR>(ls);
+                    };
+                    const bool exact = first || !a.lagged_shift;
+                    float m_l = exact ? row_max(v2) : lse_slot[g0 / GR];
+                    float s_sum = shifted_exps(m_l, v2);
+                    if (!exact && !__all(s_sum >= 0x1p-30f && s_sum <= 0x1p30f)) {
+                        // v2 again, opaque to the compiler: kept from sharing the first
+                        // pass's products, whose registers the exponentials then reuse
+                        float v2r[PL];
 #pragma unroll
-            for (int q = 0; q < kDeltaPrefetch; ++q) {
-                const int g = lane + q * kWave;
-                if (g < G) {
-                    float d = __uint_as_float(static_cast<unsigned>(dpre[q]));
-                    if (static_cast<unsigned>(dpre[q] >> 32) != (a.tag_base | unsigned(t - 1)))
-                        d = collect(ds + g, a.tag_base | unsigned(t - 1), a.spin_limit, a.status, dead, a.mark);
-                    gmax = OpMaxNan{}(gmax, d);
-                }
-            }
-            for (int g = lane + kDeltaPrefetch * kWave; g < G; g += kWave)
-                gmax = OpMaxNan{}(gmax, collect(ds + g, a.tag_base | unsigned(t - 1), a.spin_limit, a.status,
-                                                dead, a.mark));
-            gmax = wave_reduce(gmax, OpMaxNan{});
-            if (lane == 0) scratch[0] = gmax;
-        }
-        if (__syncthreads_or(low)) {
-            // Exact column LSE of K + u_t over the element's rows: max, then sum.
-            float cm[PL];
-#pragma unroll
-            for (int e = 0; e < PL; ++e) cm[e] = -FLT_MAX;
-#pragma unroll
-            for (int k = 0; k < RPW; ++k) {
-                const int l = wave + kWaves * k;
-                if (row0 + l >= rend) continue;
-                const float u = lds_u[cur * ROWS + l];
-#pragma unroll
-                for (int e = 0; e < PL; ++e)
-                    if (R::valid(lane, e, a.N)) cm[e] = fmaxf(cm[e], fmaf(x[k][e], ks_it, u));
-            }
-            tree_combine<VEC, CH>(cm, part, a.N, OpMax{});
-            unsigned long long* fslot = a.fxchg + size_t(cur) * 2 * G * a.N;
-            if (wave == 0) {
-                unsigned long long* mine = fslot + size_t(gid) * a.N;
-#pragma unroll
-                for (int k = 0; k < CH; ++k)
-#pragma unroll
-                    for (int q = 0; q < VEC; ++q) {
-                        const int col = R::col(lane, k) + q;
-                        if (col < a.N) publish(mine + col, cm[k * VEC + q], a.tag_base | unsigned(t), local);
+                        for (int e = 0; e < PL; ++e) {
+                            v2r[e] = v2[e];
+                            asm volatile("" : "+v"(v2r[e]));
+                        }
+                        m_l = row_max(v2r);
+                        s_sum = shifted_exps(m_l, v2r);
                     }
-            }
-            __syncthreads();
-            for (int w2 = wave; w2 < a.W; w2 += kWaves) {
-                float got[PL];
-                collect_row<VEC, CH>(fslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
-                                     a.spin_limit, a.status, dead, got, a.mark);
-                R::store(part + w2 * a.N, lane, a.N, got);
-            }
-            __syncthreads();
-            for (int j = threadIdx.x; j < a.N; j += kThreads) {
-                float mx = -FLT_MAX;
-                for (int w2 = 0; w2 < a.W; ++w2) mx = fmaxf(mx, part[w2 * a.N + j]);
-                lds_mx[j] = mx;
-            }
-            __syncthreads();
-            float mxl[PL], sm[PL];
-            R::load(lds_mx, lane, a.N, mxl, 0.0f);
+                    const float s_l = fmaxf(s_sum, sk::kSumFloor);
+                    const float lga_l = lga_slot[g0 / GR];
+                    const float lg2 = __builtin_amdgcn_logf(s_l);  // log2
+                    const float lse = m_l + lg2;
+                    lse_slot[g0 / GR] = lse;
+                    const float u_l = lga_l - kLn2 * lse;
+                    const float w_l = __builtin_amdgcn_exp2f(fmaf(lga_l, kLog2E, -lg2));  // a / s
 #pragma unroll
-            for (int e = 0; e < PL; ++e) sm[e] = 0.0f;
+                    for (int r = 0; r < GR; ++r) {
+                        const float wr = read_lane(w_l, lane_of_slot<GR>(r));
+                        uk[g0 + r] = read_lane(u_l, lane_of_slot<GR>(r));
 #pragma unroll
-            for (int k = 0; k < RPW; ++k) {
-                const int l = wave + kWaves * k;
-                if (row0 + l >= rend) continue;
-                const float u = lds_u[cur * ROWS + l];
-#pragma unroll
-                for (int e = 0; e < PL; ++e)
-                    if (R::valid(lane, e, a.N)) sm[e] += safe_exp(fmaf(x[k][e], ks_it, u) - mxl[e]);
-            }
-            tree_combine<VEC, CH>(sm, part, a.N);
-            unsigned long long* sslot = fslot + size_t(G) * a.N;
-            if (wave == 0) {
-                unsigned long long* mine = sslot + size_t(gid) * a.N;
-#pragma unroll
-                for (int k = 0; k < CH; ++k)
-#pragma unroll
-                    for (int q = 0; q < VEC; ++q) {
-                        const int col = R::col(lane, k) + q;
-                        if (col < a.N) publish(mine + col, sm[k * VEC + q], a.tag_base | unsigned(t), local);
+                        for (int e = 0; e < PL; ++e) acc[e] = fmaf(y[r][e], wr, acc[e]);
                     }
-            }
-            __syncthreads();
-            for (int w2 = wave; w2 < a.W; w2 += kWaves) {
-                float got[PL];
-                collect_row<VEC, CH>(sslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
-                                     a.spin_limit, a.status, dead, got, a.mark);
-                R::store(part + w2 * a.N, lane, a.N, got);
-            }
-            __syncthreads();
-            for (int j = threadIdx.x; j < a.N; j += kThreads) {
-                const float vj = lds_v[cur * a.N + j];
-                if (vj != vj) {
-                    float s = 0.0f;
-                    for (int w2 = 0; w2 < a.W; ++w2) s += part[w2 * a.N + j];
-                    lds_v[cur * a.N + j] = lds_lb[j] - (lds_mx[j] + logf(fmaxf(s, sk::kSumFloor)));
+                    // Materialise acc here: left alone, the compiler postpones the updates
+                    // to the end of the loop and keeps every group's exponentials live.
+#pragma unroll
+                    for (int e = 0; e < PL; ++e) asm volatile("" : "+v"(acc[e]));
                 }
+                float dmax = 0.0f;
+#pragma unroll
+                for (int k = 0; k < RPW; ++k) {
+                    const int l = wave + kWaves * k;
+                    const int i = row0 + l;
+                    if (i < rend) {
+                        dmax = fmaxf(dmax, fabsf(uk[k] - lds_u[prev * ROWS + l]));
+                        if (lane == 0) {
+                            lds_u[cur * ROWS + l] = uk[k];
+                            if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + i] = uk[k];
+                        }
+                    }
+                }
+                // The last readers of part (the previous exchange or exact fallback)
+                // are behind the barrier that ends the previous iteration's exchange.
+                R::store(part + wave * a.N, lane, a.N, acc);
+                if (lane == 0) scratch[1 + wave] = dmax;
+                __syncthreads();
+                if (check && threadIdx.x == 0) publish_delta(t);
+                exchange_columns<kColRounds<PL>>(
+                    part, a.xchg + size_t(cur) * G * a.N, a.N, b, a.W, w, a.tag_base | unsigned(t), local, a.spin_limit,
+                    a.status, dead, a.mark,
+                    [&](int j, float cs) {
+                        if (cs >= sk::kColSumFloor && cs <= FLT_MAX) {
+                            lds_v[cur * a.N + j] = lds_lb[j] + lds_v[prev * a.N + j] - logf(cs);
+                        } else {
+                            lds_v[cur * a.N + j] = __builtin_nanf("");  // exact LSE below
+                            low = 1;
+                        }
+                    });
+                if (test && wave == 0) finish_deltas(t, dpre);
+                first = false;
             }
-            __syncthreads();
+            resume = false;
+            if (__syncthreads_or(low)) {
+                // Exact column LSE of K + u_t over the element's rows: max, then sum.
+                float cm[PL];
+#pragma unroll
+                for (int e = 0; e < PL; ++e) cm[e] = -FLT_MAX;
+#pragma unroll
+                for (int k = 0; k < RPW; ++k) {
+                    const int l = wave + kWaves * k;
+                    if (row0 + l >= rend) continue;
+                    const float u = lds_u[cur * ROWS + l];
+#pragma unroll
+                    for (int e = 0; e < PL; ++e)
+                        if (R::valid(lane, e, a.N)) cm[e] = fmaxf(cm[e], fmaf(x[k][e], ks_it, u));
+                }
+                tree_combine<VEC, CH>(cm, part, a.N, OpMax{});
+                unsigned long long* fslot = a.fxchg + size_t(cur) * 2 * G * a.N;
+                if (wave == 0) {
+                    unsigned long long* mine = fslot + size_t(gid) * a.N;
+#pragma unroll
+                    for (int k = 0; k < CH; ++k)
+#pragma unroll
+                        for (int q = 0; q < VEC; ++q) {
+                            const int col = R::col(lane, k) + q;
+                            if (col < a.N) publish(mine + col, cm[k * VEC + q], a.tag_base | unsigned(t), local);
+                        }
+                }
+                __syncthreads();
+                for (int w2 = wave; w2 < a.W; w2 += kWaves) {
+                    float got[PL];
+                    collect_row<VEC, CH>(fslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
+                                         a.spin_limit, a.status, dead, got, a.mark);
+                    R::store(part + w2 * a.N, lane, a.N, got);
+                }
+                __syncthreads();
+                for (int j = threadIdx.x; j < a.N; j += kThreads) {
+                    float mx = -FLT_MAX;
+                    for (int w2 = 0; w2 < a.W; ++w2) mx = fmaxf(mx, part[w2 * a.N + j]);
+                    lds_mx[j] = mx;
+                }
+                __syncthreads();
+                float mxl[PL], sm[PL];
+                R::load(lds_mx, lane, a.N, mxl, 0.0f);
+#pragma unroll
+                for (int e = 0; e < PL; ++e) sm[e] = 0.0f;
+#pragma unroll
+                for (int k = 0; k < RPW; ++k) {
+                    const int l = wave + kWaves * k;
+                    if (row0 + l >= rend) continue;
+                    const float u = lds_u[cur * ROWS + l];
+#pragma unroll
+                    for (int e = 0; e < PL; ++e)
+                        if (R::valid(lane, e, a.N)) sm[e] += safe_exp(fmaf(x[k][e], ks_it, u) - mxl[e]);
+                }
+                tree_combine<VEC, CH>(sm, part, a.N);
+                unsigned long long* sslot = fslot + size_t(G) * a.N;
+                if (wave == 0) {
+                    unsigned long long* mine = sslot + size_t(gid) * a.N;
+#pragma unroll
+                    for (int k = 0; k < CH; ++k)
+#pragma unroll
+                        for (int q = 0; q < VEC; ++q) {
+                            const int col = R::col(lane, k) + q;
+                            if (col < a.N) publish(mine + col, sm[k * VEC + q], a.tag_base | unsigned(t), local);
+                        }
+                }
+                __syncthreads();
+                for (int w2 = wave; w2 < a.W; w2 += kWaves) {
+                    float got[PL];
+                    collect_row<VEC, CH>(sslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
+                                         a.spin_limit, a.status, dead, got, a.mark);
+                    R::store(part + w2 * a.N, lane, a.N, got);
+                }
+                __syncthreads();
+                for (int j = threadIdx.x; j < a.N; j += kThreads) {
+                    const float vj = lds_v[cur * a.N + j];
+                    if (vj != vj) {
+                        float s = 0.0f;
+                        for (int w2 = 0; w2 < a.W; ++w2) s += part[w2 * a.N + j];
+                        lds_v[cur * a.N + j] = lds_lb[j] - (lds_mx[j] + logf(fmaxf(s, sk::kSumFloor)));
+                    }
+                }
+                __syncthreads();
+            }
+            if (a.v_hist && w == 0)
+                for (int j = threadIdx.x; j < a.N; j += kThreads)
+                    a.v_hist[(size_t(t - 1) * a.B + b) * a.N + j] = lds_v[cur * a.N + j];
+            if (test && scratch[0] < a.tol) {  // the stop test of iteration t-1 fired
+                used = t - 1;
+                conv = 1;
+                break;
+            }
+            R::load(lds_v + cur * a.N, lane, a.N, v, 0.0f);
         }
-        if (a.v_hist && w == 0)
-            for (int j = threadIdx.x; j < a.N; j += kThreads)
-                a.v_hist[(size_t(t - 1) * a.B + b) * a.N + j] = lds_v[cur * a.N + j];
-        if (test && scratch[0] < a.tol) {  // the stop test of iteration t-1 fired
-            used = t - 1;
-            conv = 1;
-            break;
-        }
-        R::load(lds_v + cur * a.N, lane, a.N, v, 0.0f);
     }
     if (check && conv == 0 && a.max_iter >= 1) {
         if (global_delta(a, a.max_iter, scratch, dead) < a.tol) conv = 1;  // the last iteration
@@ -1108,17 +1258,36 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     const bool failed = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= a.mark;
     float vf[PL];
     R::load(lds_v + par * a.N, lane, a.N, vf, 0.0f);
-    if (a.v_out && w == 0 && wave == 0) R::store(a.v_out + bN, lane, a.N, vf);
+    if (a.v_out && w == 0)
+        for (int j = threadIdx.x; j < a.N; j += kThreads) {
+            const float vj = lds_v[par * a.N + j];
+            a.v_out[bN + j] = scal ? logf(vj) : vj;
+        }
     const float csign = a.scores_kind < 0 ? 1.0f : -1.0f;  // C = -log_alpha
     float cacc = 0.0f;
+    int row0f = row0;  // opaque, as in load_scores
+    asm volatile("" : "+s"(row0f));
 #pragma unroll
     for (int k = 0; k < RPW; ++k) {
         const int l = wave + kWaves * k;
-        const int i = row0 + l;
+        const int i = row0f + l;
+        const float wi = read_lane(w_l, lane_of_slot<RPW>(k));
         if (i >= rend) continue;
         const float ui = lds_u[par * ROWS + l];
         if (a.u_out && lane == 0) a.u_out[bM + i] = ui;
         float pv[PL];
+        if (scal) {  // P = E w V; the cost needs the scores again
+            float c[PL];
+            if (a.cost) R::load(a.X + (bM + i) * a.N, lane, a.N, c, 0.0f);
+#pragma unroll
+            for (int e = 0; e < PL; ++e) {
+                pv[e] = (x[k][e] * wi) * vf[e];
+                if (a.cost) cacc = fmaf(pv[e], csign * c[e], cacc);
+                if (failed) pv[e] = __builtin_nanf("");
+            }
+            if (a.plan) R::store(a.plan + (bM + i) * a.N, lane, a.N, pv);
+            continue;
+        }
 #pragma unroll
         for (int e = 0; e < PL; ++e) {
             const float lp = (x[k][e] * a.kscale + ui) + vf[e];

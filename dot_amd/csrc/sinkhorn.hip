@@ -472,6 +472,8 @@ bool launch_resident_forward(const dot_sinkhorn_fwd_args* a, const FwdLayout& L,
     // DOT_AMD_EXACT_ROWMAX=1: every row update shifts by the row maximum
     const char* exact_max = std::getenv("DOT_AMD_EXACT_ROWMAX");
     r.lagged_shift = (exact_max && exact_max[0] == '1') ? 0 : 1;
+    // the scaling domain needs one K scale, and log P needs the scores
+    r.scaling = (r.lagged_shift && !ks_dev && !ret_log) ? 1 : 0;
     bool ok = false;
     dispatch_resident<true>(rc, [&](auto vc, auto cc, auto rr) {
         constexpr int V = decltype(vc)::value;

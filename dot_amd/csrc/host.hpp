@@ -92,6 +92,10 @@ int sinkhorn_forward_scheduled(const dot_sinkhorn_fwd_args* a, const float* ks_h
 // negative size.  Defined in sinkhorn.hip.
 size_t forward_workspace_base_bytes(int B, int M, int N, int max_iter);
 
+// Clears 32-bit words with a kernel on the stream (not a memset: a captured
+// call records it).  Defined in sinkhorn.hip.
+void fill_zero_words(void* p, size_t words, hipStream_t stream);
+
 // sweep_strip_rows, or the value of DOT_AMD_ROWS when set (tuning only).
 inline int tuned_strip_rows(int B, int M) {
     static const int forced = [] {

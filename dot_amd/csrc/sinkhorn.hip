@@ -13,6 +13,8 @@
 #include "persistent.cuh"
 #include "resident.cuh"
 #include "sinkhorn_kernels.cuh"
+#include "tiled.cuh"
+#include "tiled.hpp"
 #include "wide.cuh"
 
 namespace dot_amd {
@@ -192,7 +194,11 @@ __global__ void fill_value(float* p, size_t n, float value) {
         p[i] = value;
 }
 
-void launch_fill_zero(void* p, size_t words, hipStream_t stream) {
+void launch_fill_zero(void* p, size_t words, hipStream_t stream) { fill_zero_words(p, words, stream); }
+
+}  // namespace
+
+void fill_zero_words(void* p, size_t words, hipStream_t stream) {
     if (words == 0) return;
     ProfScope prof("dot_fill_zero", stream);
     if (reinterpret_cast<uintptr_t>(p) % 16 == 0) {
@@ -205,6 +211,8 @@ void launch_fill_zero(void* p, size_t words, hipStream_t stream) {
     hipLaunchKernelGGL(sk::fill_zero, dim3(blocks), dim3(kBlock), 0, stream,
                        static_cast<uint32_t*>(p), words);
 }
+
+namespace {
 
 // Caller-owned exchange words of the register-resident kernels (the
 // `exchange` fields): word 0 is the status, whose failure mark is the call's
@@ -361,6 +369,64 @@ float* scaled_kernel(const dot_sinkhorn_fwd_args* a, const FwdLayout& L) {
     const size_t ek = scaled_kernel_bytes(a->B, a->M, a->N);
     if (ek == 0 || !a->workspace || a->workspace_bytes < L.bytes + ek) return nullptr;
     return reinterpret_cast<float*>(static_cast<char*>(a->workspace) + L.bytes);
+}
+
+// Exchange words of the tiled forward; in the workspace query, behind the
+// scaled kernel's room (a workspace without them takes the next tier).
+size_t tiled_bytes(int B, int M, int N) {
+    if (resident_config<true>(B, M, N, N % 4 == 0).ok) return 0;
+    const TiledCfg tc = tiled_config(B, M, N);
+    return tc.ok ? (tiled_forward_bytes(tc, B, M, N) + 255) & ~size_t(255) : 0;
+}
+
+// Launch of the tiled forward: plan wanted (it holds E meanwhile), one K
+// scale, not log P.  False when it does not take the call.
+bool try_tiled_forward(const dot_sinkhorn_fwd_args* a, const FwdLayout& L, float kscale, float log_a_default,
+                       float log_b_default, bool keep, bool vec4, hipStream_t stream) {
+    const char* env = std::getenv("DOT_AMD_PERSISTENT");
+    if (env && env[0] == '0') return false;
+    const int B = a->B, M = a->M, N = a->N;
+    const TiledCfg tc = tiled_config(B, M, N);
+    // Where the row tier keeps up per iteration, the tiles' setup (E is formed and
+    // stored once) has to pay: rows of 1025-2048 gain 4 us per iteration and cost
+    // 24 us (16 x 1024 x 2048); rows of 2049-4096 gain nothing per iteration while
+    // the row tier fills the chip, and take the tiles for their stop test alone.
+    const bool row_tier_full = int64_t(B) * pst::kMaxGroups >= device_cus();
+    if (tc.C > 1 && N <= kMaxRowLen && row_tier_full && a->max_iter < (N <= 2048 ? 8 : 32)) return false;
+    if (N > 2048 && N <= kMaxRowLen && row_tier_full && !(a->tol > 0.0f)) return false;
+    if (!tc.ok || !a->plan || a->plan == a->scores || a->max_iter < 1 || !a->workspace) return false;
+    const size_t off = L.bytes + scaled_kernel_bytes(B, M, N);
+    if (a->workspace_bytes < off + tiled_forward_bytes(tc, B, M, N)) return false;
+    til::FwdArgs r{};
+    r.X = a->scores;
+    r.kscale = kscale;
+    r.scores_kind = a->scores_kind;
+    r.log_a = a->log_a;
+    r.log_b = a->log_b;
+    r.log_a_default = log_a_default;
+    r.log_b_default = log_b_default;
+    r.tol = a->tol;
+    r.max_iter = a->max_iter;
+    r.plan = a->plan;
+    r.u_out = a->u_out;
+    r.v_out = a->v_out;
+    r.u_hist = keep ? a->u_hist : nullptr;
+    r.v_hist = keep ? a->v_hist : nullptr;
+    r.iters_used = a->iters_used;
+    r.converged = a->converged;
+    r.B = B;
+    r.M = M;
+    r.N = N;
+    r.spin_limit = spin_limit();
+    r.local_ok = local_exchange_allowed();
+    float* partial = nullptr;
+    if (!launch_tiled_forward(r, tc, vec4, a->cost != nullptr, static_cast<char*>(a->workspace) + off, &partial, stream))
+        return false;
+    if (a->cost) {
+        ProfScope prof("sk_batch_sum", stream);
+        hipLaunchKernelGGL(sk::batch_sum, dim3(B), dim3(kWave), 0, stream, partial, tc.ST * tc.C, 1.0f, a->cost);
+    }
+    return true;
 }
 
 bool launch_stream_forward(const dot_sinkhorn_fwd_args* a, const FwdLayout& L, const StreamCfg& sc,
@@ -643,7 +709,7 @@ using namespace dot_amd;
 extern "C" size_t dot_sinkhorn_forward_workspace_bytes(int B, int M, int N, int max_iter, int flags) {
     (void)flags;
     if (B < 0 || M < 0 || N < 0 || max_iter < 0) return 0;
-    return fwd_layout(nullptr, B, M, N, max_iter).bytes + scaled_kernel_bytes(B, M, N);
+    return fwd_layout(nullptr, B, M, N, max_iter).bytes + scaled_kernel_bytes(B, M, N) + tiled_bytes(B, M, N);
 }
 
 extern "C" size_t dot_sinkhorn_exchange_bytes(void) {
@@ -706,6 +772,10 @@ int dot_amd::sinkhorn_forward_scheduled(const dot_sinkhorn_fwd_args* a, const fl
                                          stream))
         return check_launch("dot_sinkhorn_forward");
     (void)hipGetLastError();  // a refused cooperative launch falls back to the next tier
+    if (!ks_dev && !ret_log &&
+        try_tiled_forward(a, L, kscale, log_a_default, log_b_default, keep, vec4, stream))
+        return check_launch("dot_sinkhorn_forward");
+    (void)hipGetLastError();
     const StreamCfg sc = stream_config(B, M, N);
     if (sc.ok && launch_stream_forward(a, L, sc, kscale, ks_dev, log_a_default, log_b_default, keep, ret_log,
                                        vec4, scaled_kernel(a, L), stream))

@@ -1,0 +1,113 @@
+"""The tiled persistent forward (row and column tiles of each element over many
+workgroups) against the float64 oracle: tile edges, rows in registers, in LDS
+and streamed, one tile per row and sixteen, and elements that leave the scaling
+domain."""
+
+import numpy as np
+import pytest
+import torch
+
+from dot_amd import _ops
+from oracle import sinkhorn as osk
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+TOL = 1e-5  # fp32 potentials of size |K| <= 100 round at 8e-6
+
+
+def _t(x):
+    return None if x is None else torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).to(DEV)
+
+
+def _run(la, tau, T, lga=None, lgb=None, tol=0.0, keep=True):
+    out = _ops.fused.sinkhorn_forward(_t(la), 1, tau, T, tol, _t(lga), _t(lgb), True, keep)
+    torch.cuda.synchronize()
+    return out
+
+
+def _check(la, tau, T, lga=None, lgb=None, tol=0.0, pick=slice(None)):
+    """Plan, cost and potentials of the elements `pick` against the oracle at the run's own count."""
+    P, cost, counts, uh, vh = _run(la, tau, T, lga, lgb, tol)
+    used = int(counts[0])
+    at = lambda x: None if x is None else x[pick]
+    ref = osk.dual_forward(la[pick], tau, used, log_a=at(lga), log_b=at(lgb), keep_history=True)
+    assert torch.isfinite(P).all()
+    P = P.cpu().numpy()[pick]
+    assert np.abs(P - ref.P).max() < TOL * np.abs(ref.P).max()
+    want = -(ref.P * la[pick]).sum((1, 2))
+    assert np.abs(cost.cpu().numpy()[pick] - want).max() < TOL * np.abs(want).max()
+    scale = max(np.abs(ref.u_hist).max(), np.abs(ref.v_hist).max())  # u + K + v rounds at its largest term
+    for got, w in ((uh, ref.u_hist), (vh, ref.v_hist)):
+        assert np.abs(got[:used].cpu().numpy()[:, pick] - w).max() < TOL * scale
+    return used
+
+
+@pytest.mark.parametrize("B,M,N", [
+    (1, 8, 1028), (1, 9, 2048), (2, 300, 2052), (3, 130, 4096), (1, 257, 4095), (2, 70, 5000), (1, 9, 16384),
+    (1, 40, 8193), (3, 300, 1001), (64, 250, 1100), (100, 150, 600), (130, 260, 512), (200, 301, 450), (90, 180, 515),
+    (256, 200, 480),
+])
+def test_matches_oracle(B, M, N):
+    print(f"tiled B={B} M={M} N={N}", flush=True)
+    rng = np.random.default_rng(B + M + N)
+    la = -rng.random((B, M, N)).astype(np.float32)
+    lga = np.log(rng.dirichlet(np.ones(M), B)).astype(np.float32).clip(-16)
+    lgb = np.log(rng.dirichlet(np.ones(N), B)).astype(np.float32).clip(-16)
+    pick = slice(None) if B * M * N < 1 << 21 else [0, B - 1]
+    assert _check(la, 0.1, 7, pick=pick) == 7
+    assert _check(la, 0.07, 4, lga, lgb, pick=pick) == 4
+    assert _check(la, 0.5, 100, tol=1e-5, pick=pick) < 100
+
+
+@pytest.mark.parametrize("B,M,N", [(3, 96, 1536), (2, 40, 4500), (40, 300, 480)])
+@pytest.mark.parametrize("far,tau", [(0.7, 0.01), (0.25, 0.004)])
+def test_leaves_at_once(B, M, N, far, tau):
+    """A far column in one element: past the bounds of V, or its sum below the floor."""
+    rng = np.random.default_rng(9)
+    la = -(0.1 * rng.random((B, M, N))).astype(np.float32)
+    la[1, :, N - 7] = -far
+    assert _check(la, tau, 8, pick=[0, 1]) == 8
+
+
+@pytest.mark.parametrize("tol", [0.0, 1e-6])
+@pytest.mark.parametrize("M,N", [(150, 1400), (90, 5000)])
+def test_leaves_after_some_iterations(M, N, tol):
+    """Two blocks whose masses do not match: the factors drift until they pass the bounds."""
+    B = 2
+    rng = np.random.default_rng(4)
+    la = -rng.random((B, M, N)).astype(np.float32)
+    la[0, : M // 2, N // 2:] -= 6.0
+    la[0, M // 2:, : N // 2] -= 6.0
+    a = np.full((B, M), 1.0)
+    a[0, : M // 2] = 9.0
+    lga = np.log(a / a.sum(1, keepdims=True)).astype(np.float32)
+    _check(la, 0.1, 45, lga=lga, tol=tol)
+
+
+def test_masked_entries_and_repeat():
+    """-inf scores, and the same bits from a second run."""
+    rng = np.random.default_rng(3)
+    la = -rng.random((2, 70, 1300)).astype(np.float32)
+    la[rng.random(la.shape) < 0.3] = -np.inf
+    idx = np.arange(1300)
+    la[:, idx % 70, idx] = -0.1
+    P, _, _, uh, vh = _run(la, 0.2, 20)
+    ref = osk.dual_forward(la, 0.2, 20)
+    assert np.abs(P.cpu().numpy() - ref.P).max() < TOL * ref.P.max()
+    Q, _, _, uh2, vh2 = _run(la, 0.2, 20)
+    assert torch.equal(P, Q) and torch.equal(uh, uh2) and torch.equal(vh, vh2)
+
+
+@pytest.mark.parametrize("env", [{"DOT_AMD_TILED": "0"}, {"DOT_AMD_AGENT_SCOPE": "1"}])
+def test_same_stop_count_as_the_row_tier(env, monkeypatch):
+    """The stop test fires at the same iteration on the row-streaming tier; the
+    exchange scope changes no bit."""
+    rng = np.random.default_rng(5)
+    la = -rng.random((3, 200, 2100)).astype(np.float32)
+    P, _, counts, _, _ = _run(la, 0.3, 200, tol=1e-5, keep=False)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    Q, _, other, _, _ = _run(la, 0.3, 200, tol=1e-5, keep=False)
+    assert abs(int(counts[0]) - int(other[0])) <= (1 if "DOT_AMD_TILED" in env else 0)
+    if "DOT_AMD_AGENT_SCOPE" in env:
+        assert torch.equal(P, Q)

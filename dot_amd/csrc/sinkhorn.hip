@@ -108,6 +108,8 @@ struct ImpLayout {
     float *r, *rs, *lam, *c, *cs, *mu, *partA, *partB, *tau_partial;
     float2* rpart;             // rows longer than kMaxRowLen: [B, nchunks, M] prologue row partials
     float* dpart;              // ... and [B, nchunks, M] row partials of each sweep
+    wide::ImpStop* stop;       // ... and [B] stop states, then the count of elements left
+    int* left;
     unsigned long long* xchg;  // resident path: tagged exchange slots, then status
     int* status;
     size_t groups;             // workgroups the slots are laid out for
@@ -135,6 +137,8 @@ ImpLayout imp_layout(void* ws, int B, int M, int N) {
     L.tau_partial = c.take<float>(size_t(B) * std::max(size_t(L.nstrips) * L.nchunks, size_t(pst::kMaxGroups)));
     L.rpart = c.take<float2>(L.nchunks > 1 ? size_t(B) * L.nchunks * M : 0);
     L.dpart = c.take<float>(L.nchunks > 1 ? size_t(B) * L.nchunks * M : 0);
+    L.stop = c.take<wide::ImpStop>(L.nchunks > 1 ? size_t(B) + 1 : 0);
+    L.left = reinterpret_cast<int*>(L.stop ? L.stop + B : nullptr);
     // The resident path runs at most one workgroup per CU and only for N <= 1024.
     const size_t groups = resident_groups_max(B, M, N);
     // [2, G, N] sweep slots, [2, G, N] prologue slots, [2, G] result words, then the status word
@@ -1107,10 +1111,24 @@ bool launch_stream_adjoint(const dot_sinkhorn_bwd_args* a, const ImpLayout& L, c
 // fold, then per sweep a rows pass (chunk partials of P mu), a columns pass
 // (lambda and the column partials of P lambda) and the mu combine, then the
 // gradient in chunk tiles.
-void launch_wide_implicit(const dot_sinkhorn_bwd_args* a, const ImpLayout& L, const sk::ImpArgs& x,
-                          float inv_tau, hipStream_t stream) {
+// Without DOT_SK_EXACT_SWEEPS an element's sweeps end once sk::AdjointStop finds
+// them converged (its workgroups then return at once), and the launches end
+// once every element has: the count of elements left is read back after sweeps
+// 4, 6, ..., 16, 32, 64, ... (a wait on the stream each, ~20 us against the 95 us
+// of a sweep at 4 x 1024 x 16384; not on a stream under capture).
+int launch_wide_implicit(const dot_sinkhorn_bwd_args* a, const ImpLayout& L, const sk::ImpArgs& x,
+                         float inv_tau, hipStream_t stream) {
     const int B = a->B, M = a->M, N = a->N;
+    int rc = DOT_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool early = !(a->flags & DOT_SK_EXACT_SWEEPS) && a->iters > 1;
+    const bool read_back = early && hipStreamIsCapturing(stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
     wide::ImpArgs w{};
+    if (early) {
+        w.stop = L.stop;
+        w.left = L.left;
+        launch_fill_zero(L.stop, size_t(B) * sizeof(wide::ImpStop) / sizeof(uint32_t), stream);
+    }
     w.s = x;
     w.rpart = L.rpart;
     w.dpart = L.dpart;
@@ -1131,6 +1149,7 @@ void launch_wide_implicit(const dot_sinkhorn_bwd_args* a, const ImpLayout& L, co
             hipLaunchKernelGGL(wide::imp_row_totals, dim3(row_blocks), dim3(kBlock), 0, stream, w);
             hipLaunchKernelGGL(sk::imp_prep_combine, sk::fold_grid(N, B), dim3(kBlock), 0, stream, x);
         }
+        if (early) hipLaunchKernelGGL(wide::imp_stop_init, dim3(1), dim3(1), 0, stream, w);
         for (int it = 0; it < a->iters; ++it) {
             {
                 ProfScope prof("sk_imp_wide_rows", stream);
@@ -1140,11 +1159,30 @@ void launch_wide_implicit(const dot_sinkhorn_bwd_args* a, const ImpLayout& L, co
                 ProfScope prof("sk_imp_wide_cols", stream);
                 hipLaunchKernelGGL((wide::imp_cols<V, C>), tiles, dim3(kBlock), lds, stream, w);
             }
-            {
+            if (!early) {
                 ProfScope prof("sk_imp_combine", stream);
                 hipLaunchKernelGGL(sk::imp_mu_combine, sk::fold_grid(N, B), dim3(kBlock), 0, stream, x);
+                continue;
+            }
+            const int t = it + 1;
+            {
+                ProfScope prof("sk_imp_combine", stream);
+                hipLaunchKernelGGL(wide::imp_mu_track, sk::fold_grid(N, B), dim3(kBlock), 0, stream, w, t);
+                hipLaunchKernelGGL(wide::imp_stop, batch_grid(1, B), dim3(kWave), 0, stream, w, t);
+            }
+            if (read_back && t >= 4 && t < a->iters && (t <= 16 ? t % 2 == 0 : (t & (t - 1)) == 0)) {
+                int left = 0;
+                if (hipMemcpyAsync(&left, L.left, sizeof(left), hipMemcpyDeviceToHost, stream) != hipSuccess ||
+                    hipStreamSynchronize(stream) != hipSuccess) {
+                    rc = fail(DOT_ERR_HIP, "dot_sinkhorn_backward_implicit: stop-count read failed");
+                    return;
+                }
+                if (left == 0) break;
             }
         }
+        if (early && a->sweeps_used)
+            hipLaunchKernelGGL(wide::imp_sweeps, dim3(unsigned(std::min((B + kBlock - 1) / kBlock, 1024))),
+                               dim3(kBlock), 0, stream, w, a->iters, a->sweeps_used);
         {
             ProfScope prof("sk_imp_final", stream);
             hipLaunchKernelGGL((wide::imp_final<V, C>), tiles, dim3(kBlock), 0, stream, w);
@@ -1155,6 +1193,7 @@ void launch_wide_implicit(const dot_sinkhorn_bwd_args* a, const ImpLayout& L, co
                                -inv_tau, a->grad_tau, nullptr, a->status);
         }
     });
+    return rc;
 }
 
 // The whole reverse pass as one cooperative launch when every batch element
@@ -1336,9 +1375,9 @@ extern "C" int dot_sinkhorn_backward_implicit(const dot_sinkhorn_bwd_args* a, do
         if (int e = check_launch("dot_sinkhorn_backward_implicit")) return e;
         (void)hipGetLastError();
     }
-    report_all_sweeps(a, stream);  // the per-sweep launches run every sweep
+    report_all_sweeps(a, stream);  // (rows longer than kMaxRowLen may end early and then report their own)
     if (L.nchunks > 1) {
-        launch_wide_implicit(a, L, x, inv_tau, stream);
+        if (int e = launch_wide_implicit(a, L, x, inv_tau, stream)) return e;
         return check_launch("dot_sinkhorn_backward_implicit");
     }
     bool launched = dispatch_row(N, bwd_vec4(a), [&](auto vc, auto cc) {

@@ -194,11 +194,25 @@ __global__ __launch_bounds__(kBlock) void materialize(sk::MaterializeArgs a, int
 // -------------------------------------------------------------------------
 // Implicit adjoint
 // -------------------------------------------------------------------------
+// The early end of an element's sweeps (sk::AdjointStop) between launches.  The
+// maxima of a sweep's change and operand size are spread over kStripes words
+// (a word each for all workgroups serialises their atomics), by sweep parity.
+constexpr int kStripes = kWave;
+struct ImpStop {
+    unsigned change[2][kStripes];  // bits of max |mu_t - mu_{t-1}|
+    unsigned scale[2][kStripes];   // bits of max (|c_k| + |sum_i P lambda_i|) / cs_k
+    sk::AdjointStop rule;
+    int done;                      // sweeps run once converged; 0 before
+};
+
 struct ImpArgs {
     sk::ImpArgs s;     // r, rs, lam, c, cs, mu, partA/B ([B,nstrips,N]), grad, tau_partial, ...
     float2* rpart;     // [B,nchunks,M]: chunk sums of P G and P (prologue)
     float* dpart;      // [B,nchunks,M]: chunk sums of P mu (each sweep)
+    ImpStop* stop;     // [B], cleared; null: every sweep runs
+    int* left;         // elements still sweeping
     int B, nchunks;
+    __device__ __forceinline__ bool ended(int b) const { return stop && stop[b].done != 0; }
 };
 
 // Prologue: chunk partials of r_i = sum_k P G and rs_i = sum_k P, and the
@@ -264,7 +278,7 @@ static __global__ __launch_bounds__(kBlock) void imp_row_totals(ImpArgs w) {
 template <int VEC, int CH>
 __global__ __launch_bounds__(kBlock) void imp_rows(ImpArgs w) {
     const int b = batch_of_block();
-    if (b >= w.B) return;
+    if (b >= w.B || w.ended(b)) return;
     using R = Row<VEC, CH>;
     const sk::ImpArgs& a = w.s;
     const Tile tl = tile_of_block(w.nchunks, a.N);
@@ -293,7 +307,7 @@ __global__ __launch_bounds__(kBlock) void imp_rows(ImpArgs w) {
 template <int VEC, int CH>
 __global__ __launch_bounds__(kBlock) void imp_cols(ImpArgs w) {
     const int b = batch_of_block();
-    if (b >= w.B) return;
+    if (b >= w.B || w.ended(b)) return;
     using R = Row<VEC, CH>;
     const sk::ImpArgs& a = w.s;
     extern __shared__ float lds[];
@@ -318,6 +332,59 @@ __global__ __launch_bounds__(kBlock) void imp_cols(ImpArgs w) {
     }
     block_column_combine<VEC, CH>(acc, lds, tl.nc);
     if (wave == 0) R::store(a.partA + (size_t(b) * a.nstrips + tl.s) * a.N + tl.c0, lane, tl.nc, acc);
+}
+
+// Sweep t, mu: as sk::imp_mu_combine, with this sweep's change and operand size
+// for the stop test.
+static __global__ __launch_bounds__(kBlock) void imp_mu_track(ImpArgs w, int t) {
+    const int b = batch_of_block();
+    if (b >= w.B || w.ended(b)) return;
+    const sk::ImpArgs& a = w.s;
+    const float* planes[1] = {a.partA};
+    float sum[1];
+    sk::fold_strips<1>(planes, a.nstrips, a.N, b, sum);
+    if (threadIdx.x >= kWave) return;  // the first wave holds the columns (fold_lane() == 0)
+    const int j = sk::fold_col();
+    float d = 0.0f, scale = 0.0f;
+    if (sk::fold_lane() == 0 && j < a.N) {
+        const size_t bj = size_t(b) * a.N + j;
+        const float c = a.c[bj], cs = fmaxf(a.cs[bj], kSumFloor);
+        const float m = (c - sum[0]) / cs;
+        d = fabsf(m - a.mu[bj]);
+        scale = (fabsf(c) + fabsf(sum[0])) / cs;
+        a.mu[bj] = m;
+    }
+    d = wave_max(d);
+    scale = wave_max(scale);
+    if (threadIdx.x == 0) {
+        const int q = int(blockIdx.x) % kStripes;
+        atomicMax(&w.stop[b].change[t & 1][q], __float_as_uint(d));
+        atomicMax(&w.stop[b].scale[t & 1][q], __float_as_uint(scale));
+    }
+}
+
+// After sweep t: the stop test of each element (a wave each), and the words of
+// the next sweep cleared.
+static __global__ __launch_bounds__(kWave) void imp_stop(ImpArgs w, int t) {
+    const int b = batch_of_block();
+    if (b >= w.B || w.ended(b)) return;
+    ImpStop& st = w.stop[b];
+    const int cur = t & 1, lane = threadIdx.x;
+    const float d = wave_max(__uint_as_float(st.change[cur][lane]));
+    const float s = wave_max(__uint_as_float(st.scale[cur][lane]));
+    st.change[cur ^ 1][lane] = st.scale[cur ^ 1][lane] = 0u;
+    if (lane == 0 && st.rule.done(t, d, s)) {
+        st.done = t;
+        atomicAdd(w.left, -1);
+    }
+}
+
+static __global__ void imp_stop_init(ImpArgs w) { *w.left = w.B; }
+
+// The sweeps each element ran.
+static __global__ void imp_sweeps(ImpArgs w, int iters, int32_t* out) {
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < w.B; b += gridDim.x * blockDim.x)
+        out[b] = w.stop[b].done ? w.stop[b].done : iters;
 }
 
 // grad = P (G - lambda_i - mu_k) / tau and per-tile sums of grad * log_alpha,

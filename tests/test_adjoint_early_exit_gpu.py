@@ -226,3 +226,30 @@ def test_persistent_slabs_beyond_the_cus(monkeypatch):
     res_x, g_x = _run(C, tau, T, BT, _t(a), _t(b))
     assert res_x.adjoint_sweeps == [BT] * B
     assert rel_err(g, g_x.cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("B,M,N,tau,BT,nonuni", [
+    (1, 40, 4097, 0.3, 60, False),
+    (3, 70, 5000, 0.5, 90, True),
+    (2, 33, 8192, 0.1, 100, False),
+    (2, 64, 4500, 0.2, 3, True),
+])
+def test_long_rows_end_early(B, M, N, tau, BT, nonuni, monkeypatch):
+    """Rows longer than 4096 columns (a launch per pass and sweep): early end
+    against every sweep and the float64 oracle at the full count."""
+    print(f"[early-end] long rows B={B} M={M} N={N} tau={tau} BT={BT}", flush=True)
+    rng = np.random.default_rng(B * 1000 + M + N)
+    Cn = rng.random((B, M, N)).astype(np.float32)
+    a = _dirichlet(rng, B, M) if nonuni else None
+    b = _dirichlet(rng, B, N) if nonuni else None
+    lt = lambda x: None if x is None else _t(x)
+    res, g = _run(_t(Cn), tau, 30, BT, lt(a), lt(b))
+    sweeps = res.adjoint_sweeps
+    monkeypatch.setenv("DOT_AMD_EXACT_SWEEPS", "1")
+    full, gf = _run(_t(Cn), tau, 30, BT, lt(a), lt(b))
+    assert full.adjoint_sweeps == [BT] * B
+    assert all(1 <= q <= BT for q in sweeps) and (BT < 10 or max(sweeps) < BT)
+    _, want = _oracle_grad(Cn, tau, 30, BT, a, b)
+    scale = np.abs(want).max()
+    assert np.abs(g.cpu().numpy() - want).max() < 1e-4 * scale
+    assert np.abs(gf.cpu().numpy() - want).max() < 1e-4 * scale

@@ -333,6 +333,15 @@ __device__ __forceinline__ int logical_group(int W) {
     return blockIdx.x;
 }
 
+// The same for a grid that may be padded to 8 ceil(B / 8) W workgroups
+// (padded_groups): element e then gets W blocks of XCD e mod 8, and a
+// workgroup without an element (-1) returns at once.
+__device__ __forceinline__ int logical_group(int W, int G) {
+    if (int(gridDim.x) == G) return logical_group(W);
+    const int e = int(blockIdx.x % kXcds) + kXcds * int(blockIdx.x / kXcds / W);
+    return e * W < G ? e * W + int(blockIdx.x / kXcds) % W : -1;
+}
+
 // Element q of a small per-thread array through static indices only (a
 // dynamic index would place the array in scratch memory, and every reload
 // from there waits for all memory operations in flight).
@@ -455,6 +464,7 @@ struct ImpResArgs {
     float* grad_tau;           // [B] out: tau_scale * sum(grad * log_alpha)
     float tau_scale;
     unsigned long long* rwords;  // [2, G] tagged result words: grad_tau partials, failure flags
+    int G;                     // workgroups with an element (the grid may be padded)
     unsigned result_tag;
     int32_t* status_out;       // the caller's status word (1: a wait gave up), or null
     int keep_status;           // nonzero: raise status_out only (a later slab of one call)
@@ -512,8 +522,9 @@ __global__ __launch_bounds__(kThreads) void implicit_adjoint(ImpResArgs a) {
     float* stopbuf = scratch + kWaves;
     const int lane = threadIdx.x % kWave;
     const int wave = threadIdx.x / kWave;
-    const int G = gridDim.x;
-    const int gid = logical_group(a.W);
+    const int G = a.G;
+    const int gid = logical_group(a.W, G);
+    if (gid < 0) return;
     const int b = gid / a.W;
     const int w = gid % a.W;
     const int row0 = w * a.R;
@@ -727,7 +738,7 @@ struct FwdResArgs {
     unsigned long long* fxchg;  // [2, 2, G, N] tagged exact-fallback column max / sum
     unsigned long long* dxchg;  // [kDeltaSlots, G] tagged per-workgroup deltas
     int* status;                // at least `mark` after a poll timeout of this call
-    int B, M, N, W, R, spin_limit;
+    int B, M, N, W, R, G, spin_limit;  // G: workgroups with an element (the grid may be padded)
     unsigned tag_base;          // exchange tags are tag_base | t (0: slots cleared for the call)
     unsigned xcc_tag;           // tag of the XCD-id words
     int mark;                   // failure mark in *status (forced_timeout)
@@ -751,7 +762,7 @@ constexpr float kScaledColMin = 0x1p-50f;
 // must call it; wave 0 polls.
 __device__ __forceinline__ float global_delta(const FwdResArgs& a, int t, float* scratch, bool& dead) {
     const int lane = threadIdx.x % kWave;
-    const int G = gridDim.x;
+    const int G = a.G;
     __syncthreads();
     if (threadIdx.x < kWave) {
         unsigned long long* ds = a.dxchg + size_t(t % kDeltaSlots) * G;
@@ -782,6 +793,16 @@ __device__ __forceinline__ float global_delta(const FwdResArgs& a, int t, float*
 // update and reads them after the exchange, so the test costs no wait of its
 // own; when it fires, iteration t is discarded and (u_{t-1}, v_{t-1}) are the
 // result.
+
+// |u_t - u_{t-1}| of a row in the scaling domain, for the stop test: ln(w_t /
+// w_{t-1}) by its series once the factors agree to 1 %, which resolves changes
+// down to the rounding of the row's sum (~1e-7); the difference of the two
+// rounded potentials (one unit in the last place is 4e-6 at |u| = 40) before.
+__device__ __forceinline__ float scaled_change(float w, float w_prev, float u, float u_prev) {
+    const float x = (w - w_prev) / w_prev;
+    return fabsf(x) <= 0.01f ? fabsf(x - 0.5f * x * x) : fabsf(u - u_prev);
+}
+
 constexpr int kDeltaPrefetch = 4;  // delta loads in flight per lane of wave 0 (covers 256 workgroups)
 
 template <int VEC, int CH, int RPW, bool SCHED = false>
@@ -801,8 +822,9 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     float* scratch = lds_la + ROWS;  // [0] global delta, [1..kWaves] wave deltas, [16..] reductions
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // row addresses in scalar registers
-    const int G = gridDim.x;
-    const int gid = logical_group(a.W);
+    const int G = a.G;
+    const int gid = logical_group(a.W, G);
+    if (gid < 0) return;
     const int b = gid / a.W;
     const int w = gid % a.W;
     const int row0 = w * a.R;
@@ -977,7 +999,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
 #pragma unroll
                 for (int e = 0; e < PL; ++e) acc[e] = fmaf(x[k][e], wk, acc[e]);
             }
-            if (check) dmax = wave_max(row_ok ? fabsf(u_l - u_prev) : 0.0f);
+            if (check) dmax = wave_max(row_ok ? scaled_change(w_l, w_prev, u_l, u_prev) : 0.0f);
             u_prev = u_l;
             if (row_owner) {
                 lds_u[cur * ROWS + lslot] = u_l;
@@ -1305,7 +1327,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
             if (w == 0) a.cost[b] = s;
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (gid == 0 && threadIdx.x == 0) {
         *a.iters_used = failed ? -1 : used;  // -1: an exchange timed out, the outputs are NaN
         *a.converged = conv;
     }

@@ -306,6 +306,16 @@ ResidentCfg resident_config(int B, int M, int N, bool vec4) {
     return c;
 }
 
+// Workgroups to launch for B elements of W: when they do not split evenly over
+// the XCDs, 8 ceil(B / 8) W if every XCD's share then fits its CUs, so that an
+// element's workgroups share an XCD (12 x 700 x 500, W = 6: the exchange words
+// stay in its L2) and the padding returns at once.
+int padded_groups(int B, int W) {
+    const int per_xcd = (B + res::kXcds - 1) / res::kXcds * W;
+    const bool even = (B * W) % res::kXcds == 0 && (B * W / res::kXcds) % W == 0;
+    return W > 1 && !even && per_xcd <= device_cus() / res::kXcds ? per_xcd * res::kXcds : B * W;
+}
+
 template <bool Forward, class F>
 bool dispatch_resident(const ResidentCfg& c, F&& f) {
     constexpr bool Fwd = Forward;
@@ -537,6 +547,7 @@ bool launch_resident_forward(const dot_sinkhorn_fwd_args* a, const FwdLayout& L,
     r.N = a->N;
     r.W = rc.W;
     r.R = rc.R;
+    r.G = groups;
     r.spin_limit = spin_limit();
     r.local_ok = local_exchange_allowed();
     // DOT_AMD_EXACT_ROWMAX=1: every row update shifts by the row maximum
@@ -562,8 +573,8 @@ bool launch_resident_forward(const dot_sinkhorn_fwd_args* a, const FwdLayout& L,
         // one workgroup per element exchanges only with itself; the stop test
         // (tol > 0) couples all workgroups of the batch
         const bool independent = rc.W == 1 && (!(a->tol > 0.0f) || groups == 1);
-        ok = launch_grid(reinterpret_cast<const void*>(kernel), groups, res::kThreads, params, lds, stream,
-                         independent) == hipSuccess;
+        ok = launch_grid(reinterpret_cast<const void*>(kernel), padded_groups(a->B, rc.W), res::kThreads, params,
+                         lds, stream, independent) == hipSuccess;
     });
     return ok;
 }
@@ -979,6 +990,7 @@ bool launch_resident_adjoint(const dot_sinkhorn_bwd_args* a, const ImpLayout& L,
     r.N = a->N;
     r.W = rc.W;
     r.R = rc.R;
+    r.G = groups;
     r.iters = a->iters;
     r.spin_limit = spin_limit();
     r.local_ok = local_exchange_allowed();
@@ -1002,8 +1014,8 @@ bool launch_resident_adjoint(const dot_sinkhorn_bwd_args* a, const ImpLayout& L,
         ProfScope prof("sk_imp_resident", stream);
         // the adjoint's exchanges stay within a batch element's W workgroups,
         // but the status word waits for the whole grid
-        ok = launch_grid(reinterpret_cast<const void*>(kernel), groups, res::kThreads, params, lds, stream,
-                         rc.W == 1 && !a->status) == hipSuccess;
+        ok = launch_grid(reinterpret_cast<const void*>(kernel), padded_groups(a->B, rc.W), res::kThreads, params,
+                         lds, stream, rc.W == 1 && !a->status) == hipSuccess;
     });
     return ok;
 }

@@ -15,9 +15,15 @@
 namespace dot_amd {
 namespace {
 
-// Column chunks of a row: 1 when a row fits a wave's registers, else rows
-// are swept in wide::kChunk-column tiles (bidi_wide.cuh).
-int row_chunks(int L2) { return L2 > kMaxRowLen ? wide::num_chunks(L2) : 1; }
+// Column chunks of a row: 1 up to 1024 columns (bidi_kernels.cuh), else the
+// rows are swept in tiles of 1024 (bidi_wide.cuh).  A whole row per wave takes
+// 32 floats per lane from 1025 columns on and 64 from 2049: the two row buffers
+// and the column state then leave one or two waves per SIMD, and a small batch
+// gets strips of four rows, whose column partials are half a read of the
+// matrix.  Forward and backward, whole rows -> tiles: 3 x 2100 x 2900 536 ->
+// 131 us, 3 x 2100 x 2901 (ragged) 1737 -> 106, 16 x 1024 x 2048 234 -> 197,
+// 12 x 1300 x 1500 221 -> 164, 1 x 100 x 1400 91 -> 53, 20 x 2048 x 1056 328 -> 326.
+int row_chunks(int L2) { return bidi::wide_rows::num_chunks(L2); }
 
 int strip_rows_bidi(int B, int L1, int nchunks) {
     static const int forced = [] {
@@ -34,6 +40,7 @@ size_t lds_bytes(int N) { return (size_t(2) * N + 8) * sizeof(float); }
 
 // ---- one-pass tier (bidi_onepass.cuh)
 namespace op = bidi::onepass;
+using bidi::wide_rows::kCols;
 static_assert(op::kMaxEpoch == DOT_BIDISOFTMAX_MAX_EPOCH, "epoch limit of the header");
 
 // Groups of 32 workgroups: one per XCD (32 CUs each on gfx950), at most 8.
@@ -241,29 +248,29 @@ extern "C" int dot_bidisoftmax_forward(const dot_bidisoftmax_fwd_args* a, dot_st
         w.B = B;
         w.nchunks = L.nchunks;
         const dim3 tiles = batch_grid(unsigned(L.nstrips) * unsigned(L.nchunks), B);
-        const unsigned row_blocks = unsigned((size_t(B) * L1 + kWavesPerBlock - 1) / kWavesPerBlock);
-        wide::dispatch_chunk(vec4, [&](auto vc, auto cc) {
+        const bidi::wide_rows::FoldGrid fold(L1, L2);
+        bidi::wide_rows::dispatch(vec4, [&](auto vc, auto cc) {
             constexpr int V = decltype(vc)::value;
             constexpr int C = decltype(cc)::value;
             {
                 ProfScope prof("bidi_fwd_stats", stream);
                 hipLaunchKernelGGL((bidi::wide_rows::fwd_stats<V, C>), tiles, dim3(kBlock),
-                                   lds_bytes(wide::kChunk), stream, w);
+                                   lds_bytes(kCols), stream, w);
             }
             {
                 ProfScope prof("bidi_fwd_col_combine", stream);
-                hipLaunchKernelGGL(bidi::wide_rows::fwd_row_stats, dim3(row_blocks), dim3(kBlock), 0, stream, w);
-                hipLaunchKernelGGL(bidi::fwd_col_combine, fold_grid, dim3(kBlock), 0, stream, x);
+                hipLaunchKernelGGL(bidi::wide_rows::fwd_fold, batch_grid(unsigned(fold.cols + fold.rows), B),
+                                   dim3(kBlock), 0, stream, w, fold.cols);
             }
             {
                 ProfScope prof("bidi_fwd_write", stream);
                 hipLaunchKernelGGL((bidi::wide_rows::fwd_write<V, C>), tiles, dim3(kBlock),
-                                   2 * size_t(wide::kChunk) * sizeof(float), stream, w);
+                                   (2 * size_t(kCols) + 2 * L.rows) * sizeof(float), stream, w);
             }
         });
         return check_launch("dot_bidisoftmax_forward");
     }
-    bool launched = dispatch_row(L2, vec4, [&](auto vc, auto cc) {
+    bool launched = dispatch_row<kCols>(L2, vec4, [&](auto vc, auto cc) {
         constexpr int V = decltype(vc)::value;
         constexpr int C = decltype(cc)::value;
         {
@@ -368,8 +375,8 @@ extern "C" int dot_bidisoftmax_backward(const dot_bidisoftmax_bwd_args* a, dot_s
         w.B = B;
         w.nchunks = L.nchunks;
         const dim3 tiles = batch_grid(unsigned(L.nstrips) * unsigned(L.nchunks), B);
-        const unsigned row_blocks = unsigned((size_t(B) * L1 + kWavesPerBlock - 1) / kWavesPerBlock);
-        wide::dispatch_chunk(vec4, [&](auto vc, auto cc) {
+        const bidi::wide_rows::FoldGrid fold(L1, L2);
+        bidi::wide_rows::dispatch(vec4, [&](auto vc, auto cc) {
             constexpr int V = decltype(vc)::value;
             constexpr int C = decltype(cc)::value;
             auto run = [&](auto recompute) {
@@ -377,19 +384,18 @@ extern "C" int dot_bidisoftmax_backward(const dot_bidisoftmax_bwd_args* a, dot_s
                 {
                     ProfScope prof("bidi_bwd_dots", stream);
                     hipLaunchKernelGGL((bidi::wide_rows::bwd_dots<V, C, RC>), tiles, dim3(kBlock),
-                                       2 * size_t(wide::kChunk) * sizeof(float) + lds_bytes(wide::kChunk),
+                                       (2 * size_t(kCols) + 2 * L.rows) * sizeof(float) + lds_bytes(kCols),
                                        stream, w);
                 }
                 {
                     ProfScope prof("bidi_bwd_fold", stream);
-                    hipLaunchKernelGGL(bidi::wide_rows::bwd_row_dots, dim3(row_blocks), dim3(kBlock), 0, stream, w);
-                    hipLaunchKernelGGL(bidi::column_fold, fold_grid, dim3(kBlock), 0, stream, L.partial, L.nstrips,
-                                       B, L2, L.dot_c);
+                    hipLaunchKernelGGL(bidi::wide_rows::bwd_fold, batch_grid(unsigned(fold.cols + fold.rows), B),
+                                       dim3(kBlock), 0, stream, w, fold.cols);
                 }
                 {
                     ProfScope prof("bidi_bwd_write", stream);
                     hipLaunchKernelGGL((bidi::wide_rows::bwd_write<V, C, RC>), tiles, dim3(kBlock),
-                                       3 * size_t(wide::kChunk) * sizeof(float), stream, w);
+                                       (3 * size_t(kCols) + 3 * L.rows) * sizeof(float), stream, w);
                 }
             };
             if (buffers) run(std::false_type{});
@@ -402,7 +408,7 @@ extern "C" int dot_bidisoftmax_backward(const dot_bidisoftmax_bwd_args* a, dot_s
         }
         return check_launch("dot_bidisoftmax_backward");
     }
-    bool launched = dispatch_row(L2, vec4, [&](auto vc, auto cc) {
+    bool launched = dispatch_row<kCols>(L2, vec4, [&](auto vc, auto cc) {
         constexpr int V = decltype(vc)::value;
         constexpr int C = decltype(cc)::value;
         auto run = [&](auto recompute) {

@@ -166,10 +166,8 @@ __global__ __launch_bounds__(kBlock) void fwd_stats(FwdArgs a) {
 constexpr int kFoldCols = 16;
 constexpr int kFoldLanes = kBlock / kFoldCols;  // 16
 
-static __global__ __launch_bounds__(kBlock) void fwd_col_combine(FwdArgs a) {
+__device__ __forceinline__ void col_combine_block(const FwdArgs& a, int b) {
     __shared__ float sm_m[kFoldLanes][kFoldCols], sm_s[kFoldLanes][kFoldCols];
-    const int b = batch_of_block();
-    if (b >= a.B) return;
     const int jj = threadIdx.x % kFoldCols;
     const int sl = threadIdx.x / kFoldCols;
     const int j = blockIdx.x * kFoldCols + jj;
@@ -197,13 +195,15 @@ static __global__ __launch_bounds__(kBlock) void fwd_col_combine(FwdArgs a) {
     }
 }
 
+static __global__ __launch_bounds__(kBlock) void fwd_col_combine(FwdArgs a) {
+    const int b = batch_of_block();
+    if (b < a.B) col_combine_block(a, b);
+}
+
 // Column sums of the strips' partial rows, in the same fixed order as
 // fwd_col_combine.
-static __global__ __launch_bounds__(kBlock) void column_fold(const float* partial, int nstrips, int B, int N,
-                                                             float* out) {
+__device__ __forceinline__ void column_fold_block(const float* partial, int nstrips, int b, int N, float* out) {
     __shared__ float sm[kFoldLanes][kFoldCols];
-    const int b = batch_of_block();
-    if (b >= B) return;
     const int jj = threadIdx.x % kFoldCols;
     const int sl = threadIdx.x / kFoldCols;
     const int j = blockIdx.x * kFoldCols + jj;
@@ -222,6 +222,12 @@ static __global__ __launch_bounds__(kBlock) void column_fold(const float* partia
         }
     }
     if (sl == 0 && j < N) out[size_t(b) * N + j] = s;
+}
+
+static __global__ __launch_bounds__(kBlock) void column_fold(const float* partial, int nstrips, int B, int N,
+                                                             float* out) {
+    const int b = batch_of_block();
+    if (b < B) column_fold_block(partial, nstrips, b, N, out);
 }
 
 // Column max and reciprocal column sum of one batch element into LDS, shared
@@ -347,39 +353,44 @@ struct BwdRow {
         float y[R::PL], g[R::PL];
         float r[kBufPL], c[kBufPL], o[kBufPL];
     };
-    const float* lcm;   // LDS: column max (base 2), L2 floats
+    const float* lcm;   // LDS: column max (base 2), n floats
     const float* lics;  // LDS: 1 / column sum
     const float* lrm;   // LDS: row max (base 2) of the strip's rows
     const float* lirs;  // LDS: 1 / row sum
     int r0;
+    int n;   // columns of the tile (L2 when it is the whole row)
+    int nl;  // ... of which the rows' loads take the first nl (> 0; a multiple of VEC)
     float sc;
 
-    // `lds` holds 2 * L2 + 2 * rows floats; the caller places the barrier
-    // before the first get().  [r0, rv) are the strip's valid rows.
-    __device__ void init(const BwdArgs& a, int b, float* lds, int r0_, int rv) {
+    // `lds` holds 2 * n + 2 * rows floats; the caller places the barrier
+    // before the first get().  [r0, rv) are the strip's valid rows, [c0, c0 + n)
+    // the tile's columns.
+    __device__ void init(const BwdArgs& a, int b, float* lds, int r0_, int rv, int c0, int n_, int nl_) {
         sc = a.inv_T * kLog2E;
         r0 = r0_;
+        n = n_;
+        nl = nl_;
         float* cm = lds;
-        float* ics = lds + a.L2;
-        float* rm = lds + 2 * a.L2;
+        float* ics = lds + n;
+        float* rm = lds + 2 * n;
         float* irs = rm + a.rows;
         lcm = cm;
         lics = ics;
         lrm = rm;
         lirs = irs;
         if constexpr (RECOMPUTE) {
-            load_col_stats(a.col_stats + size_t(b) * 2 * a.L2, a.L2, cm, ics);
+            load_col_stats(a.col_stats + size_t(b) * 2 * a.L2 + c0, a.L2, n, cm, ics);
             load_row_stats(a.row_stats + size_t(b) * 2 * a.L1, a.L1, r0, rv, rm, irs);
         }
     }
 
     __device__ void load(const BwdArgs& a, size_t off, int lane, Buf& t) const {
-        R::load_clamped(a.sim + off, lane, a.L2, t.y, 0.0f);
-        R::load_clamped(a.grad_out + off, lane, a.L2, t.g, 0.0f);
+        R::load_clamped(a.sim + off, lane, nl, t.y, 0.0f);
+        R::load_clamped(a.grad_out + off, lane, nl, t.g, 0.0f);
         if constexpr (!RECOMPUTE) {
-            R::load(a.row_sm + off, lane, a.L2, t.r, 0.0f);
-            R::load(a.col_sm + off, lane, a.L2, t.c, 0.0f);
-            R::load(a.out + off, lane, a.L2, t.o, 0.0f);
+            R::load(a.row_sm + off, lane, nl, t.r, 0.0f);
+            R::load(a.col_sm + off, lane, nl, t.c, 0.0f);
+            R::load(a.out + off, lane, nl, t.o, 0.0f);
         }
     }
 
@@ -391,8 +402,8 @@ struct BwdRow {
 #pragma unroll
             for (int k = 0; k < CH; ++k) {
                 float cm[VEC], ics[VEC];
-                R::chunk(lcm, lane, k, a.L2, cm);
-                R::chunk(lics, lane, k, a.L2, ics);
+                R::chunk(lcm, lane, k, n, cm);
+                R::chunk(lics, lane, k, n, ics);
 #pragma unroll
                 for (int q = 0; q < VEC; ++q) {
                     const int e = k * VEC + q;
@@ -420,10 +431,10 @@ struct BwdRow {
 // of sim and grad_out); buffer mode, with five arrays per row, visits them
 // one at a time.
 template <bool RECOMPUTE, class Src, class Body>
-__device__ __forceinline__ void bwd_rows(const BwdArgs& a, const Src& src, int b, int i0, int r1, int lane,
+__device__ __forceinline__ void bwd_rows(const BwdArgs& a, const Src& src, int b, int c0, int i0, int r1, int lane,
                                          Body&& body) {
     using Buf = typename Src::Buf;
-    auto load = [&](int i, Buf& t) { src.load(a, (size_t(b) * a.L1 + i) * a.L2, lane, t); };
+    auto load = [&](int i, Buf& t) { src.load(a, (size_t(b) * a.L1 + i) * a.L2 + c0, lane, t); };
     if constexpr (RECOMPUTE) {
         pipelined_rows<Buf>(i0, r1, kWavesPerBlock, load, body);
     } else {
@@ -454,13 +465,13 @@ __global__ __launch_bounds__(kBlock) void bwd_dots(BwdArgs a) {
     const int r0 = st * a.rows;
     const int r1 = min(r0 + a.rows, l1);
     Src src;
-    src.init(a, b, lds, r0, r1);
+    src.init(a, b, lds, r0, r1, 0, a.L2, a.L2);
     __syncthreads();
     float* comb = lds + 2 * a.L2 + 2 * a.rows;
     float acc[R::PL];
 #pragma unroll
     for (int e = 0; e < R::PL; ++e) acc[e] = 0.0f;
-    bwd_rows<RECOMPUTE>(a, src, b, r0 + wave, r1, lane, [&](int i, const typename Src::Buf& t) {
+    bwd_rows<RECOMPUTE>(a, src, b, 0, r0 + wave, r1, lane, [&](int i, const typename Src::Buf& t) {
         float r[R::PL], c[R::PL], d[R::PL];
         src.get(a, i, lane, l2, full, t, r, c, d);
         float dl = 0.0f;
@@ -500,14 +511,14 @@ __global__ __launch_bounds__(kBlock) void bwd_write(BwdArgs a) {
     for (int j = threadIdx.x; j < a.L2; j += kBlock) ldc[j] = a.dot_c[size_t(b) * a.L2 + j];
     for (int t = threadIdx.x; t < rv - r0; t += kBlock) ldr[t] = a.dot_r[size_t(b) * a.L1 + r0 + t];
     Src src;
-    src.init(a, b, lds, r0, rv);
+    src.init(a, b, lds, r0, rv, 0, a.L2, a.L2);
     __syncthreads();
     float tacc = 0.0f;
     const bool want_tau = a.tau_partial != nullptr;  // null: grad_tau not requested
     auto store = [&](int i, const float(&gs)[R::PL]) {
         R::store_stream(a.grad_sim + (size_t(b) * a.L1 + i) * a.L2, lane, a.L2, gs);
     };
-    bwd_rows<RECOMPUTE>(a, src, b, r0 + wave, rv, lane, [&](int i, const typename Src::Buf& t) {
+    bwd_rows<RECOMPUTE>(a, src, b, 0, r0 + wave, rv, lane, [&](int i, const typename Src::Buf& t) {
         float r[R::PL], c[R::PL], d[R::PL], gs[R::PL];
         src.get(a, i, lane, l2, full, t, r, c, d);
         const float dr = ldr[i - r0];

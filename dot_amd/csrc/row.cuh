@@ -197,18 +197,22 @@ __device__ __forceinline__ void pipelined_rows(int i0, int r1, int step, Load&& 
 }
 
 // Pick (VEC, CH) for a row length and call f(integral_constant<VEC>, integral_constant<CH>).
-// Returns false when N is outside the register-resident range.
-template <class F>
+// Returns false when N is outside the register-resident range (MAX: 1024 where
+// the caller's kernels take longer rows in tiles, else kMaxRowLen).
+template <int MAX = kMaxRowLen, class F>
 bool dispatch_row(int N, bool vec4, F&& f) {
     using std::integral_constant;
-    if (N <= 0 || N > kMaxRowLen) return false;
+    static_assert(MAX == 1024 || MAX == kMaxRowLen, "a limit of the layouts below");
+    if (N <= 0 || N > MAX) return false;
     if (vec4) {
         const int chunks = (N + 255) / 256;
         if (chunks <= 1) f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
         else if (chunks <= 2) f(integral_constant<int, 4>{}, integral_constant<int, 2>{});
         else if (chunks <= 4) f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
-        else if (chunks <= 8) f(integral_constant<int, 4>{}, integral_constant<int, 8>{});
-        else f(integral_constant<int, 4>{}, integral_constant<int, 16>{});
+        else if constexpr (MAX > 1024) {
+            if (chunks <= 8) f(integral_constant<int, 4>{}, integral_constant<int, 8>{});
+            else f(integral_constant<int, 4>{}, integral_constant<int, 16>{});
+        }
     } else {
         const int chunks = (N + 63) / 64;
         if (chunks <= 1) f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
@@ -216,8 +220,10 @@ bool dispatch_row(int N, bool vec4, F&& f) {
         else if (chunks <= 4) f(integral_constant<int, 1>{}, integral_constant<int, 4>{});
         else if (chunks <= 8) f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
         else if (chunks <= 16) f(integral_constant<int, 1>{}, integral_constant<int, 16>{});
-        else if (chunks <= 32) f(integral_constant<int, 1>{}, integral_constant<int, 32>{});
-        else f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
+        else if constexpr (MAX > 1024) {
+            if (chunks <= 32) f(integral_constant<int, 1>{}, integral_constant<int, 32>{});
+            else f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
+        }
     }
     return true;
 }

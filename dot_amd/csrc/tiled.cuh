@@ -371,6 +371,13 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
             setup(x, k, y);
             if (k + KB < nk) setup(y, k + KB, x);
         }
+    } else {  // a wave without rows adds 0 w = 0 to the column sums: its registers must not hold infinities or NaN
+#pragma unroll
+        for (int q = 0; q < RR / KB; ++q)
+#pragma unroll
+            for (int r = 0; r < KB; ++r)
+#pragma unroll
+                for (int e = 0; e < PL; ++e) xr[q][r][e] = 0.0f;
     }
 
     // XCD checks: the words of a row stay in its strip, those of a column in its tiles

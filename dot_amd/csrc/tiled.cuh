@@ -564,7 +564,8 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
         bool left = leave, bad = false;
         clear();
         if (leave) {
-            for (int l = threadIdx.x; l < nrows; l += kThreads)
+            // (a row of one tile has no row words: everyone who would read them leaves as well)
+            for (int l = threadIdx.x; C > 1 && l < nrows; l += kThreads)
                 publish(rowx + (bM + row0 + l) * C + c, INFINITY, tag);
         } else {
             float v[PL];

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import dot_amd
-from dot_amd import _ops
+from dot_amd import _ops, profiler
 from oracle import sinkhorn as osk
 
 pytestmark = pytest.mark.gpu
@@ -126,3 +126,38 @@ def test_waves_without_rows(B, M, N):
         if want is None:
             want = res.transport_plan
         assert torch.equal(res.transport_plan, want), k
+
+
+@pytest.mark.parametrize("B,M,N", [(144, 400, 450), (100, 150, 600)])
+def test_leaving_elements_touch_no_neighbour(B, M, N):
+    """One tile per row: every third element leaves the scaling domain, at an
+    iteration of its own.  The others keep the bits that they have beside a
+    batch in which none leaves, and a second run has the same bits."""
+    T = 24
+    rng = np.random.default_rng(B)
+    calm = -rng.random((B, M, N)).astype(np.float32)
+    a = np.full((B, M), 1.0)
+    la, lga0 = calm.copy(), np.log(a / M).astype(np.float32)
+    for e in range(0, B, 3):
+        la[e, : M // 2, N // 2:] -= 6.0
+        la[e, M // 2:, : N // 2] -= 6.0
+        a[e, : M // 2] = (9.0, 30.0, 100.0)[e // 3 % 3]
+    lga = np.log(a / a.sum(1, keepdims=True)).astype(np.float32)
+    profiler.reset()
+    profiler.enable(True, ["sk_fwd_tiled"])
+    try:
+        got = _run(la, 0.1, T, lga)
+        profiler.collect()
+        assert profiler.query("sk_fwd_tiled")[0] == 1
+    finally:
+        profiler.enable(False)
+    again, alone = _run(la, 0.1, T, lga), _run(calm, 0.1, T, lga0)
+    assert int(got[2][0]) == T
+    for e in range(0, B, 3):  # a potential beyond 40 ln 2 = 27.7 has left, and none starts there
+        assert got[4][0, e].abs().max() < 27 < 28 < got[4][-1, e].abs().max()
+    rest = [e for e in range(B) if e % 3]
+    for k, dim in ((0, 0), (3, 1), (4, 1)):  # plan, u and v histories
+        assert torch.equal(got[k], again[k])
+        pick = torch.tensor(rest, device=DEV)
+        assert torch.equal(got[k].index_select(dim, pick), alone[k].index_select(dim, pick))
+    assert _check(la, 0.1, T, lga, pick=[0, 1, 3, 6, B - 1]) == T

@@ -794,13 +794,15 @@ __device__ __forceinline__ float global_delta(const FwdResArgs& a, int t, float*
 // own; when it fires, iteration t is discarded and (u_{t-1}, v_{t-1}) are the
 // result.
 
-// |u_t - u_{t-1}| of a row in the scaling domain, for the stop test: ln(w_t /
-// w_{t-1}) by its series once the factors agree to 1 %, which resolves changes
-// down to the rounding of the row's sum (~1e-7); the difference of the two
-// rounded potentials (one unit in the last place is 4e-6 at |u| = 40) before.
+// |u_t - u_{t-1}| of a row in the scaling domain, for the stop test: |ln(w_t /
+// w_{t-1})|, by its series once the factors agree to 1 %.  It resolves changes
+// down to the rounding of the row's sum (~2e-7), which the difference of two
+// rounded potentials does not (one unit in the last place is 4e-6 at |u| = 40,
+// 1024 in a row of scores of -1e9 at reg 0.1).
 __device__ __forceinline__ float scaled_change(float w, float w_prev, float u, float u_prev) {
     const float x = (w - w_prev) / w_prev;
-    return fabsf(x) <= 0.01f ? fabsf(x - 0.5f * x * x) : fabsf(u - u_prev);
+    if (fabsf(x) <= 0.01f) return fabsf(x - 0.5f * x * x);
+    return w_prev > 0.0f ? fabsf(kLn2 * __builtin_amdgcn_logf(w / w_prev)) : fabsf(u - u_prev);
 }
 
 constexpr int kDeltaPrefetch = 4;  // delta loads in flight per lane of wave 0 (covers 256 workgroups)

@@ -34,10 +34,10 @@
 // that iteration's rows in the log domain, from the scores.
 //
 // The stop test sees |u_t - u_{t-1}| as ln(w_t / w_{t-1}), resolved to the
-// rounding of a row's sum, so it fires where 64-bit arithmetic has it fire (25 x
-// 670 x 1651 at reg 0.987: iteration 3; the rounded potentials wobble by more
-// than tol = 1e-6 and ran all 262).  Where a potential's own float spacing
-// exceeds tol it does not fire: potentials of that size cannot show the change.
+// rounding of a row's sum (~2e-7) whatever the size of the potentials, so it
+// fires where 64-bit arithmetic has it fire (25 x 670 x 1651 at reg 0.987:
+// iteration 3; the rounded potentials wobble by more than tol = 1e-6 and ran
+// all 262).
 #pragma once
 
 #include <cfloat>
@@ -221,12 +221,6 @@ struct RowGroup {
     }
 };
 
-// The first power of two whose float spacing exceeds tol.
-__device__ __forceinline__ float spacing_limit(float tol) {
-    const float x = tol * 0x1p23f;
-    return x < 0x1p-100f ? 0x1p-100f : __uint_as_float((__float_as_uint(x) & 0x7f800000u) + 0x800000u);
-}
-
 template <int VEC, int CH, int KB, int RR>
 __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     using Rw = Row<VEC, CH>;
@@ -275,7 +269,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
         lds_la[l] = la;
         lds_row4[l] = make_float4(exp_compensated(la), 0.0f, 0.0f, 0.0f);
     }
-    const float limit = spacing_limit(a.tol);
     for (int j = threadIdx.x; j < nc; j += kThreads) {
         lds_lb[j] = a.log_b ? a.log_b[bN + c0 + j] : a.log_b_default;
         lds_v[j] = lds_v[seg + j] = 1.0f;
@@ -402,7 +395,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     bool leave = false;  // ... until the next iteration's row update
     int used = a.max_iter;
     int conv = 0;
-    int coarse = -1;  // whether a potential's spacing exceeds tol (-1: not looked at)
     float acc[PL], dmax = 0.0f;
     auto clear = [&]() {
         dmax = 0.0f;
@@ -466,21 +458,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
             float d = scratch[1];
 #pragma unroll
             for (int q = 1; q < kWaves; ++q) d = fmaxf(d, scratch[1 + q]);
-            if (SC && d < a.tol) {
-                // a potential whose own spacing exceeds tol cannot show a change below it,
-                // and counts as changing, as the rounded potentials of the log domain do
-                // (looked at once: changes below tol do not move a potential's size)
-                if (coarse < 0) {
-                    bool any = false;
-                    for (int l = threadIdx.x; l < nrows; l += kThreads) {
-                        const float4 q = lds_row4[l];
-                        const float wl = cur ? q.w : q.z;
-                        any = any || (wl > 0.0f && q.y > -FLT_MAX && fabsf(u_of(wl, q.y)) >= limit);
-                    }
-                    coarse = __syncthreads_or(any) ? 1 : 0;
-                }
-                if (coarse) d = INFINITY;
-            }
             if (threadIdx.x == 0) publish(a.dxchg + size_t(t % res::kDeltaSlots) * G + gid, d, tag);
         }
 
@@ -602,7 +579,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 bad = bad || (ok && !(s_sum == 0.0f || (s_sum > 0.0f && w <= res::kScaleMax)));
                 if (check) {
                     // |u_t - u_{t-1}| = |ln(w_t / w_{t-1})|, by its series once the factors agree
-                    // to 1 %: resolved to the rounding of the row's sum (~1e-7).  A row without
+                    // to 1 %: resolved to the rounding of the row's sum (~2e-7).  A row without
                     // mass or without a finite score does not count.
                     const float w_prev = cur ? rw.z : rw.w;
                     const float q = (w - w_prev) * __builtin_amdgcn_rcpf(w_prev);
@@ -610,7 +587,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                     if (__any(ok && !(fabsf(q) <= 0.01f))) {
                         if (ok && !(fabsf(q) <= 0.01f))
                             d = w > 0.0f && s_sum > 0.0f
-                                    ? fabsf(u_of(w, rw.y) - (t > 1 ? u_of(w_prev, rw.y) : 0.0f)) : 0.0f;
+                                    ? fabsf(t > 1 ? kLn2 * __builtin_amdgcn_logf(w / w_prev) : u_of(w, rw.y)) : 0.0f;
                     }
                     dmax = fmaxf(dmax, d);
                 }

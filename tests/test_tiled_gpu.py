@@ -1,6 +1,6 @@
 """The tiled persistent forward (row and column tiles of each element over many
-workgroups) against the float64 oracle: tile edges, rows in registers, in LDS
-and streamed, one tile per row and sixteen, and elements that leave the scaling
+workgroups) against the float64 oracle: tile edges, rows in registers and rows
+streamed, one tile per row and sixteen, and elements that leave the scaling
 domain."""
 
 import numpy as np
@@ -161,3 +161,45 @@ def test_leaving_elements_touch_no_neighbour(B, M, N):
         pick = torch.tensor(rest, device=DEV)
         assert torch.equal(got[k].index_select(dim, pick), alone[k].index_select(dim, pick))
     assert _check(la, 0.1, T, lga, pick=[0, 1, 3, 6, B - 1]) == T
+
+
+# (2, 200, 300) is resident, the others tiled
+@pytest.mark.parametrize("B,M,N", [(2, 200, 300), (2, 300, 1400), (3, 150, 5000), (160, 260, 400)])
+@pytest.mark.parametrize("offset,tau", [(1.0, 0.04), (2.0, 0.04)])
+def test_stops_where_64_bits_stop(B, M, N, offset, tau):
+    """The stop test does not see the rounding of the potentials (2e-6 and 4e-6 at |u| of
+    17 and 44, above tol): the run ends at the iteration whose change the oracle has
+    below tol, up to what the ratio of two row factors resolves."""
+    tol, noise = 1e-6, 5e-7
+    rng = np.random.default_rng(M + N)
+    la = -offset - rng.random((min(B, 3), M, N)).astype(np.float32)
+    lga = np.log(rng.dirichlet(np.ones(M), len(la))).astype(np.float32).clip(-16)
+    rep = -(-B // len(la))
+    full = lambda x: np.concatenate([x] * rep)[:B]
+    P, cost, counts, uh, vh = _run(full(la), tau, 60, full(lga), None, tol)
+    used = int(counts[0])
+    ref = osk.dual_forward(la, tau, 60, log_a=lga, keep_history=True)
+    assert np.abs(ref.u_hist[-1]).max() > 16
+    assert int(counts[1]) == 1 and 1 < used < 60
+    assert ref.deltas[used - 1] < tol + noise and ref.deltas[used - 2] > tol - noise
+    own = osk.dual_forward(la, tau, used, log_a=lga)
+    assert np.abs(P[: len(la)].cpu().numpy() - own.P).max() < TOL * own.P.max()
+
+
+@pytest.mark.parametrize("B,M,N", [(2, 200, 300), (2, 300, 1400), (3, 150, 5000), (160, 260, 400)])
+def test_constant_cost_converges_at_the_second_iteration(B, M, N):
+    C = torch.full((B, M, N), 50.0, device=DEV)
+    res = dot_amd.sinkhorn(C, reg=1.0, n_iters=40, tol=1e-6)
+    assert res.n_iters_used == 2 and bool(res.converged)
+    assert torch.allclose(res.transport_plan, torch.full_like(C, 1.0 / (M * N)), rtol=TOL, atol=0.0)
+
+
+@pytest.mark.parametrize("B,M,N", [(2, 200, 300), (2, 300, 1400), (3, 150, 5000)])
+def test_tol_below_what_floats_resolve(B, M, N):
+    """The run ends at its bound (or at an exact fixed point), with the bound's plan."""
+    rng = np.random.default_rng(N)
+    la = -rng.random((B, M, N)).astype(np.float32)
+    P, _, counts, _, _ = _run(la, 0.05, 40, tol=1e-9, keep=False)
+    assert 5 < int(counts[0]) <= 40
+    ref = osk.dual_forward(la, 0.05, 40)
+    assert np.abs(P.cpu().numpy() - ref.P).max() < TOL * ref.P.max()

@@ -757,6 +757,38 @@ constexpr float kScaleMax = 0x1p40f;
 constexpr float kScaleMin = 0x1p-40f;
 constexpr float kScaledColMin = 0x1p-50f;
 
+// E = 2^((x - x_max) kscale log2 e) of a row's scores x, x_max the one whose K is
+// the largest: exactly 1 there, whatever the size of the scores (of a row that
+// is masked by -1e9, K log2 e at reg 0.1 is rounded to multiples of 1024).
+struct ScaledKernel {
+    float sign, k, lo;  // K log2 e = x (k + lo), k rounded towards zero: the two products agree in sign
+    struct Row {
+        float x, m, m_lo;  // x_max, x_max k rounded, and what the rounding left out; 0, -FLT_MAX, 0 if no K is above -inf
+    };
+    __device__ __forceinline__ explicit ScaledKernel(float kscale)
+        : sign(kscale < 0.0f ? -1.0f : 1.0f), k(kscale * kLog2E), lo(rest(kscale)) {
+        if (lo * k < 0.0f) {
+            k = __uint_as_float(__float_as_uint(k) - 1u);
+            lo = rest(kscale);
+        }
+    }
+    __device__ __forceinline__ float rest(float kscale) const {
+        return fmaf(kscale, 1.92596303e-8f, fmaf(kscale, kLog2E, -k));  // (log2 e - kLog2E)
+    }
+    // `top`: the maximum of sign x over the row, from -inf
+    __device__ __forceinline__ Row row(float top) const {
+        const float x = sign * top, p = x * k;
+        if (p == -INFINITY) return {0.0f, -FLT_MAX, 0.0f};
+        return {x, p + (p - p), fmaf(x, k, -p)};  // (m: NaN for +inf)
+    }
+    // log2 of the row's sum of exp(K + v), from lg, that of the sum of E V
+    __device__ __forceinline__ float log2_sum(const Row& r, float lg) const { return r.m + (fmaf(r.x, lo, r.m_lo) + lg); }
+    // 0 where K is -inf (the padding, a mask), NaN where x is NaN
+    __device__ __forceinline__ float e(float x, const Row& r) const {
+        return __builtin_amdgcn_exp2f(fmaf(x, k, -r.m) + fmaf(x - r.x, lo, -r.m_lo));
+    }
+};
+
 // Waits for G tagged per-workgroup deltas of iteration t and returns their
 // maximum (order-free, so every workgroup gets the same value).  Every thread
 // must call it; wave 0 polls.
@@ -892,31 +924,24 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     const int lslot = wave + kWaves * slot_of_lane<RPW>(lane);
     const bool row_ok = row0 + lslot < rend;
     const bool row_owner = lane < 16 && (lane & (16 / RPW - 1)) == 0 && row_ok;
-    float m_l = 0.0f, a_l = 0.0f, w_l = 0.0f, w_prev = 0.0f, u_prev = 0.0f;
+    const ScaledKernel kernel(a.kscale);
+    float top_l = 0.0f, a_l = 0.0f, w_l = 0.0f, w_prev = 0.0f, u_prev = 0.0f;
     float b_own[kColRounds<PL>] = {};
     if constexpr (!SCHED) {
         if (scal) {
             float lm[RPW];
 #pragma unroll
             for (int k = 0; k < RPW; ++k) {
-                lm[k] = -FLT_MAX;
+                lm[k] = -INFINITY;
 #pragma unroll
-                for (int e = 0; e < PL; ++e) lm[k] = fmaxf(lm[k], x[k][e] * kscale2);
+                for (int e = 0; e < PL; ++e) lm[k] = fmaxf(lm[k], x[k][e] * kernel.sign);
             }
-            m_l = transposed_reduce<RPW>(lm, OpMax{});
-            // what the rounding of kscale log2(e) left out, times a finite x (an
-            // infinite one has its infinity from the first term already)
-            constexpr float kLog2ELo = 1.92596303e-8f;  // log2 e - kLog2E
-            const float kscale2_lo = fmaf(a.kscale, kLog2ELo, fmaf(a.kscale, kLog2E, -kscale2));
+            top_l = transposed_reduce<RPW>(lm, OpMax{});
 #pragma unroll
             for (int k = 0; k < RPW; ++k) {
-                const float m = read_lane(m_l, lane_of_slot<RPW>(k));
+                const auto row = kernel.row(read_lane(top_l, lane_of_slot<RPW>(k)));
 #pragma unroll
-                for (int e = 0; e < PL; ++e) {
-                    const float xf = fminf(fmaxf(x[k][e], -FLT_MAX), FLT_MAX);
-                    const float y = fmaf(xf, kscale2_lo, fmaf(x[k][e], kscale2, -m));
-                    x[k][e] = __builtin_amdgcn_exp2f(y);  // 0 for the padding, whose y is -inf
-                }
+                for (int e = 0; e < PL; ++e) x[k][e] = kernel.e(x[k][e], row);
             }
             a_l = exp_compensated(lds_la[lslot]);
 #pragma unroll
@@ -989,7 +1014,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
             const float s_l = s_sum > 0.0f ? s_sum : sk::kSumFloor;  // 0: a row with no finite K
             w_prev = w_l;
             w_l = a_l / s_l;
-            const float u_l = lds_la[lslot] - kLn2 * (m_l + __builtin_amdgcn_logf(s_l));
+            const float u_l = lds_la[lslot] - kLn2 * kernel.log2_sum(kernel.row(top_l), __builtin_amdgcn_logf(s_l));
             // a row factor out of range, or NaN: every column's sum becomes NaN,
             // which all workgroups of the element see
             const bool bad = __any(row_ok && s_sum != 0.0f && !(w_l <= kScaleMax));

@@ -3,7 +3,7 @@
 //
 // Workgroup (s, c) of element b owns the tile of rows [s R, (s+1) R) and
 // columns [c seg, (c+1) seg).  The iteration runs in the scaling domain of
-// res::forward: E_ij = 2^(K_ij log2(e) - m_i) once, then
+// res::forward: E_ij = 2^(K_ij log2(e) - max_j) once (res::ScaledKernel), then
 //   w_i = a_i / sum_j E_ij V_j,   V_j = b_j / sum_i E_ij w_i,   P = E w V,
 // two FMAs per element and iteration.  Each wave takes every eighth row of
 // the tile in batches of KB rows and completes a batch's row sums by itself:
@@ -57,7 +57,7 @@ typedef unsigned long long word_t;
 constexpr int kMaxTiles = 16;                 // column tiles per batch element (C)
 constexpr int kMaxStrips = 256;               // row strips per batch element (ST)
 constexpr unsigned kLogBit = 0x80000000u;     // tag bit: the word is v, not V
-constexpr unsigned kSetupTag = 0x7ffffffeu;   // row maxima (an iteration tag is below it)
+constexpr unsigned kSetupTag = 0x7ffffffeu;   // rows' largest scores (an iteration tag is below it)
 constexpr int kColsPerThread = 3;             // ceil((1024 + kMaxStrips) / kThreads)
 
 struct FwdArgs {
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     float* lds_v = fold + kWaves * seg;  // [2][seg] V by iteration parity (v in the log domain)
     float* lds_lb = lds_v + 2 * seg;
     float* red = lds_lb + seg;
-    // a row of the scaling domain: a, the row maximum m, w by iteration parity
+    // a row of the scaling domain: a, the row's largest score (times the sign of K), w by iteration parity
     float4* lds_row4 = reinterpret_cast<float4*>(lds + ((size_t(kWaves) + 3) * seg + ((seg + ST + 3) & ~3)));
     float* lds_u = reinterpret_cast<float*>(lds_row4 + R);  // log domain: u by iteration parity
     float* lds_la = lds_u + 2 * R;
@@ -308,38 +308,33 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 if (!Rw::valid(lane, e, nc)) x[r][e] = pad;
     };
 
-    // E of a batch: the row maxima over the tiles, then 2^(K log2 e - m) with the
-    // rounding of kscale log2(e) made up for (a finite score's share of it).
-    const float kscale2_lo = fmaf(a.kscale, 1.92596303e-8f, fmaf(a.kscale, kLog2E, -kscale2));
-    auto e_of = [&](float x, float m) {
-        const float xf = fminf(fmaxf(x, -FLT_MAX), FLT_MAX);
-        return __builtin_amdgcn_exp2f(fmaf(xf, kscale2_lo, fmaf(x, kscale2, -m)));
-    };
+    // E of a batch, from the rows' largest scores over the tiles
+    const res::ScaledKernel kernel(a.kscale);
     auto form_e = [&](float(&x)[KB][PL], int k0) {
         mask_rows(x);
         float lm[KB];
 #pragma unroll
         for (int r = 0; r < KB; ++r) {
-            lm[r] = -FLT_MAX;
+            lm[r] = -INFINITY;
 #pragma unroll
-            for (int e = 0; e < PL; ++e) lm[r] = fmaxf(lm[r], x[r][e] * kscale2);
+            for (int e = 0; e < PL; ++e) lm[r] = fmaxf(lm[r], x[r][e] * kernel.sign);
         }
         const float own = res::transposed_reduce<KB>(lm, OpMax{});
-        float m;
+        float top;
         if (C > 1) {
             rg.put(a.rowx, own, k0, nk, kSetupTag, false);
-            m = rg.get(a.rowx, k0, nk, kSetupTag, a.spin_limit, a.status, dead);
-            m = group_reduce(rg.reads(k0, nk) ? m : -FLT_MAX, rg.lg, OpMax{});
+            top = rg.get(a.rowx, k0, nk, kSetupTag, a.spin_limit, a.status, dead);
+            top = group_reduce(rg.reads(k0, nk) ? top : -INFINITY, rg.lg, OpMax{});
         } else {
-            m = rg.to_group(own);
+            top = rg.to_group(own);
         }
-        if (rg.leader() && rg.group_ok(k0, nk)) lds_row4[rg.group_row(k0)].y = m;
+        if (rg.leader() && rg.group_ok(k0, nk)) lds_row4[rg.group_row(k0)].y = top;
 #pragma unroll
         for (int r = 0; r < KB; ++r) {
-            const float mr = rg.of_group(m, r);
+            const auto row = kernel.row(rg.of_group(top, r));
             const bool in = k0 + r < nk;  // rows past the last: 0
 #pragma unroll
-            for (int e = 0; e < PL; ++e) x[r][e] = in ? e_of(x[r][e], mr) : 0.0f;
+            for (int e = 0; e < PL; ++e) x[r][e] = in ? kernel.e(x[r][e], row) : 0.0f;
         }
     };
 
@@ -436,7 +431,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
         publish(a.uslot + size_t(t & 1) * a.B * a.M + bM + row0 + l, u, unsigned(t));
         if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + row0 + l] = u;
     };
-    auto u_of = [&](float w, float m) { return kLn2 * (__builtin_amdgcn_logf(w) - m); };
+    auto u_of = [&](float w, float top) { return -kLn2 * kernel.log2_sum(kernel.row(top), -__builtin_amdgcn_logf(w)); };
     // the potentials of iteration t from its factors, for the log domain
     auto rows_to_u = [&](int t) {
         for (int l = threadIdx.x; l < nrows; l += kThreads) {
@@ -801,10 +796,11 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     auto write_row = [&](int l, float(&x)[PL], const float(&sc)[PL], bool from_scores, int ln) {
         const float4 q = lds_row4[l];
         const float wi = par ? q.w : q.z, ui = scal ? 0.0f : lds_u[par * R + l];
+        const auto row = kernel.row(q.y);
 #pragma unroll
         for (int e = 0; e < PL; ++e) {
             float p;
-            if (scal) p = ((from_scores ? e_of(sc[e], q.y) : x[e]) * wi) * vf[e];
+            if (scal) p = ((from_scores ? kernel.e(sc[e], row) : x[e]) * wi) * vf[e];
             else p = safe_exp((sc[e] * a.kscale + ui) + vf[e]);
             if (a.cost_partial && Rw::valid(ln, e, nc)) cacc = fmaf(p, csign * sc[e], cacc);
             x[e] = failed ? __builtin_nanf("") : p;

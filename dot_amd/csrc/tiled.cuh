@@ -29,8 +29,8 @@
 // An element leaves the scaling domain for the log domain for good when a
 // factor or a column sum passes its bounds (res::kScaleMax ...): the owner of
 // such a column forms the exact column log-sum-exp and publishes v itself
-// under a tag with kLogBit set, the workgroups that gather it publish infinite
-// row words in the next iteration, and so every workgroup of the element redoes
+// under a tag with kLogBit set, the workgroups that gather it tag their row
+// words of the next iteration with it, and so every workgroup of the element redoes
 // that iteration's rows in the log domain, from the scores.
 //
 // The stop test sees |u_t - u_{t-1}| as ln(w_t / w_{t-1}), resolved to the
@@ -56,7 +56,7 @@ typedef unsigned long long word_t;
 
 constexpr int kMaxTiles = 16;                 // column tiles per batch element (C)
 constexpr int kMaxStrips = 256;               // row strips per batch element (ST)
-constexpr unsigned kLogBit = 0x80000000u;     // tag bit: the word is v, not V
+constexpr unsigned kLogBit = 0x80000000u;     // tag bit: a column's word is v, not V; a row's tile leaves
 constexpr unsigned kSetupTag = 0x7ffffffeu;   // rows' largest scores (an iteration tag is below it)
 constexpr int kColsPerThread = 3;             // ceil((1024 + kMaxStrips) / kThreads)
 
@@ -97,15 +97,20 @@ inline __host__ __device__ size_t fwd_lds_floats(int seg, int ST, int R) {
     return ((size_t(kWaves) + 3) * seg + red + 7 * size_t(R) + 32 + 3) & ~size_t(3);
 }
 
-// Polls one tagged word per lane (lanes with `on`) until all carry tag t; NaN
-// after a timeout.  `dead` is kept uniform over the wave.
+// Polls one tagged word per lane (lanes with `on`) until all carry tag t (or t |
+// kLogBit: `left`, for the wave); NaN after a timeout.  `dead` is kept uniform
+// over the wave.
 __device__ __forceinline__ float poll_lane(const word_t* p, bool on, unsigned t, int spin_limit, int* status,
-                                           bool& dead) {
+                                           bool& dead, bool& left) {
     res::forced_timeout(spin_limit, status, dead);
     for (int spins = 0; !dead; ++spins) {
         word_t x = tag_pack(0.0f, t);
         if (on) x = __hip_atomic_load(const_cast<word_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__all(static_cast<unsigned>(x >> 32) == t)) return __uint_as_float(static_cast<unsigned>(x));
+        const unsigned tag = static_cast<unsigned>(x >> 32);
+        if (__all((tag & ~kLogBit) == t)) {
+            left = __any(tag != t);
+            return __uint_as_float(static_cast<unsigned>(x));
+        }
         const bool failed =
             (spins & 255) == 255 && __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
         if (spins >= spin_limit) atomicOr(status, 1);
@@ -204,10 +209,15 @@ struct RowGroup {
         return group_ok(k0, kend) && (lane & ((1 << lg) - 1)) < C;
     }
     __device__ __forceinline__ float get(const word_t* slots, int k0, int kend, unsigned t, int spin_limit,
-                                         int* status, bool& dead, int words = 1, int which = 0) const {
+                                         int* status, bool& dead, bool& left, int words = 1, int which = 0) const {
         return poll_lane(reinterpret_cast<const word_t*>(reinterpret_cast<const char*>(slots) +
                                                          (get_at + unsigned(k0) * step) * unsigned(words)) + which,
-                         reads(k0, kend), t, spin_limit, status, dead);
+                         reads(k0, kend), t, spin_limit, status, dead, left);
+    }
+    __device__ __forceinline__ float get(const word_t* slots, int k0, int kend, unsigned t, int spin_limit,
+                                         int* status, bool& dead, int words = 1, int which = 0) const {
+        bool left;  // (nobody leaves here)
+        return get(slots, k0, kend, t, spin_limit, status, dead, left, words, which);
     }
     // one tile per row: the value moves to its group's lane without memory
     __device__ __forceinline__ float to_group(float own) const {
@@ -538,7 +548,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
         if (leave) {
             // (a row of one tile has no row words: everyone who would read them leaves as well)
             for (int l = threadIdx.x; C > 1 && l < nrows; l += kThreads)
-                publish(rowx + (bM + row0 + l) * C + c, INFINITY, tag);
+                publish(rowx + (bM + row0 + l) * C + c, 0.0f, tag | kLogBit);
         } else {
             float v[PL];
             Rw::load(lds_v + prev * seg, lane, nc, v, 0.0f);
@@ -557,8 +567,9 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 float s_sum;
                 if (C > 1) {
                     const bool on = rg.reads(k0, nk);
-                    s_sum = rg.get(rowx, k0, nk, tag, a.spin_limit, a.status, dead);
-                    if (__any(on && s_sum == INFINITY)) {  // a peer leaves: all of the strip's rows say so
+                    bool peer_left = false;
+                    s_sum = rg.get(rowx, k0, nk, tag, a.spin_limit, a.status, dead, peer_left);
+                    if (peer_left) {  // all of the strip's rows say so
                         left = true;
                         return;
                     }

@@ -834,7 +834,8 @@ __device__ __forceinline__ float global_delta(const FwdResArgs& a, int t, float*
 __device__ __forceinline__ float scaled_change(float w, float w_prev, float u, float u_prev) {
     const float x = (w - w_prev) / w_prev;
     if (fabsf(x) <= 0.01f) return fabsf(x - 0.5f * x * x);
-    return w_prev > 0.0f ? fabsf(kLn2 * __builtin_amdgcn_logf(w / w_prev)) : fabsf(u - u_prev);
+    // (a row of a zero marginal: inf in the first iteration, the difference of two -inf does not count)
+    return w_prev > 0.0f ? fabsf(kLn2 * __builtin_amdgcn_logf(w / w_prev)) : fmaxf(fabsf(u - u_prev), 0.0f);
 }
 
 constexpr int kDeltaPrefetch = 4;  // delta loads in flight per lane of wave 0 (covers 256 workgroups)
@@ -943,11 +944,11 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
 #pragma unroll
                 for (int e = 0; e < PL; ++e) x[k][e] = kernel.e(x[k][e], row);
             }
-            a_l = exp_compensated(lds_la[lslot]);
+            a_l = safe_exp(lds_la[lslot]);
 #pragma unroll
             for (int q = 0; q < kColRounds<PL>; ++q) {
                 const int j = threadIdx.x + q * kThreads;
-                if (j < a.N) b_own[q] = exp_compensated(lds_lb[j]);
+                if (j < a.N) b_own[q] = safe_exp(lds_lb[j]);
             }
         }
     }

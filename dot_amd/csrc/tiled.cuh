@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     float* lds_v = fold + kWaves * seg;  // [2][seg] V by iteration parity (v in the log domain)
     float* lds_lb = lds_v + 2 * seg;
     float* red = lds_lb + seg;
-    // a row of the scaling domain: a, the row's largest score (times the sign of K), w by iteration parity
+    // a row of the scaling domain: a, the row's largest score (times the sign of K), sum E V by iteration parity
     float4* lds_row4 = reinterpret_cast<float4*>(lds + ((size_t(kWaves) + 3) * seg + ((seg + ST + 3) & ~3)));
     float* lds_u = reinterpret_cast<float*>(lds_row4 + R);  // log domain: u by iteration parity
     float* lds_la = lds_u + 2 * R;
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     for (int l = threadIdx.x; l < R; l += kThreads) {
         const float la = (l < nrows && a.log_a) ? a.log_a[bM + row0 + l] : a.log_a_default;
         lds_la[l] = la;
-        lds_row4[l] = make_float4(exp_compensated(la), 0.0f, 0.0f, 0.0f);
+        lds_row4[l] = make_float4(safe_exp(la), 0.0f, 0.0f, 0.0f);
     }
     for (int j = threadIdx.x; j < nc; j += kThreads) {
         lds_lb[j] = a.log_b ? a.log_b[bN + c0 + j] : a.log_b_default;
@@ -441,12 +441,15 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
         publish(a.uslot + size_t(t & 1) * a.B * a.M + bM + row0 + l, u, unsigned(t));
         if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + row0 + l] = u;
     };
-    auto u_of = [&](float w, float top) { return -kLn2 * kernel.log2_sum(kernel.row(top), -__builtin_amdgcn_logf(w)); };
-    // the potentials of iteration t from its factors, for the log domain
+    // u of a row from its sum of E V (a zero marginal's is -inf)
+    auto u_of = [&](float log_a, float top, float sum) {
+        return log_a - kLn2 * kernel.log2_sum(kernel.row(top), __builtin_amdgcn_logf(sum));
+    };
+    // the potentials of iteration t from its row sums, for the log domain
     auto rows_to_u = [&](int t) {
         for (int l = threadIdx.x; l < nrows; l += kThreads) {
             const float4 q = lds_row4[l];
-            lds_u[(t & 1) * R + l] = t > 0 ? u_of((t & 1) ? q.w : q.z, q.y) : 0.0f;
+            lds_u[(t & 1) * R + l] = t > 0 ? u_of(lds_la[l], q.y, (t & 1) ? q.w : q.z) : 0.0f;
         }
     };
     // The column sums of iteration t, exchanged into the tile's new factors:
@@ -493,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 float vn = 0.0f;
                 bool lin = SC, good;
                 if constexpr (SC) {
-                    vn = exp_compensated(lds_lb[j]) / cs;
+                    vn = safe_exp(lds_lb[j]) / cs;
                     good = cs >= res::kScaledColMin && vn >= res::kScaleMin && vn <= res::kScaleMax;
                 } else {
                     good = cs >= sk::kColSumFloor && cs <= FLT_MAX;
@@ -580,25 +583,26 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 const bool ok = rg.group_ok(k0, nk);
                 const int l = ok ? rg.group_row(k0) : 0;
                 const float4 rw = lds_row4[l];
+                const float lga = lds_la[l];
                 const float s_l = s_sum > 0.0f ? s_sum : sk::kSumFloor;  // 0: a row with no finite K
                 const float w = ok ? rw.x / s_l : 0.0f;
                 bad = bad || (ok && !(s_sum == 0.0f || (s_sum > 0.0f && w <= res::kScaleMax)));
                 if (check) {
-                    // |u_t - u_{t-1}| = |ln(w_t / w_{t-1})|, by its series once the factors agree
-                    // to 1 %: resolved to the rounding of the row's sum (~2e-7).  A row without
-                    // mass or without a finite score does not count.
-                    const float w_prev = cur ? rw.z : rw.w;
-                    const float q = (w - w_prev) * __builtin_amdgcn_rcpf(w_prev);
+                    // |u_t - u_{t-1}| = |ln(s_t / s_{t-1})|, by its series once the sums agree
+                    // to 1 %: resolved to their rounding (~2e-7).  A row of a zero marginal,
+                    // whose u is -inf, does not change after the first iteration.
+                    const float s_prev = cur ? rw.z : rw.w;
+                    const float q = (s_prev - s_l) * __builtin_amdgcn_rcpf(s_l);
                     float d = ok ? fabsf(q - 0.5f * q * q) : 0.0f;
                     if (__any(ok && !(fabsf(q) <= 0.01f))) {
                         if (ok && !(fabsf(q) <= 0.01f))
-                            d = w > 0.0f && s_sum > 0.0f
-                                    ? fabsf(t > 1 ? kLn2 * __builtin_amdgcn_logf(w / w_prev) : u_of(w, rw.y)) : 0.0f;
+                            d = fabsf(t > 1 ? kLn2 * __builtin_amdgcn_logf(s_prev / s_l) : u_of(lga, rw.y, s_l));
                     }
+                    if (t > 1 && lga == -INFINITY) d = 0.0f;
                     dmax = fmaxf(dmax, d);
                 }
-                if (c == 0 && ok && rg.leader()) put_u(t, u_of(w, rw.y), l);
-                if (ok && rg.leader()) (cur ? lds_row4[l].w : lds_row4[l].z) = w;
+                if (c == 0 && ok && rg.leader()) put_u(t, u_of(lga, rw.y, s_l), l);
+                if (ok && rg.leader()) (cur ? lds_row4[l].w : lds_row4[l].z) = s_l;
 #pragma unroll
                 for (int r = 0; r < KB; ++r) {
                     const float wr = rg.of_group(w, r);
@@ -798,7 +802,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     if (a.u_out && c == 0)
         for (int l = threadIdx.x; l < nrows; l += kThreads) {
             const float4 q = lds_row4[l];
-            a.u_out[bM + row0 + l] = scal ? u_of(par ? q.w : q.z, q.y) : lds_u[par * R + l];
+            a.u_out[bM + row0 + l] = scal ? u_of(lds_la[l], q.y, par ? q.w : q.z) : lds_u[par * R + l];
         }
     const float csign = a.scores_kind < 0 ? 1.0f : -1.0f;  // C = -log_alpha
     float cacc = 0.0f;
@@ -806,7 +810,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     // cost reads them in any case, and E need not be read as well.
     auto write_row = [&](int l, float(&x)[PL], const float(&sc)[PL], bool from_scores, int ln) {
         const float4 q = lds_row4[l];
-        const float wi = par ? q.w : q.z, ui = scal ? 0.0f : lds_u[par * R + l];
+        const float wi = q.x / (par ? q.w : q.z), ui = scal ? 0.0f : lds_u[par * R + l];
         const auto row = kernel.row(q.y);
 #pragma unroll
         for (int e = 0; e < PL; ++e) {

@@ -95,3 +95,52 @@ def test_scores_beyond_the_range_of_k(B, M, N):
     assert used == 3
     ref = osk.dual_forward(la[:1], 0.1, 3)
     assert _rel(P[:1], ref.P) < TOL
+
+
+def _marginals(B, M, N, rng, zero_rows, zero_cols):
+    """Log-marginals of which element 1 has -inf entries."""
+    a, b = rng.dirichlet(np.ones(M), B), rng.dirichlet(np.ones(N), B)
+    a[1, zero_rows] = 0.0
+    b[1, zero_cols] = 0.0
+    with np.errstate(divide="ignore"):
+        return [np.log(x / x.sum(1, keepdims=True)).astype(np.float32).clip(-16 if not z else None)
+                for x, z in ((a, len(zero_rows)), (b, len(zero_cols)))]
+
+
+@pytest.mark.parametrize("B,M,N", SHAPES)
+@pytest.mark.parametrize("rows,cols", [([3], []), ([0, 1, 7, 30], []), ([], [5]), ([2, 3, 4, 5], [0, 1, 60, 61, 62])])
+@pytest.mark.parametrize("T", [1, 2, 7])
+def test_zero_marginals(B, M, N, rows, cols, T):
+    """log a or log b of -inf: u or v of -inf, a plan of zeros there, and the
+    others' values those of the problem without these rows and columns."""
+    rng = np.random.default_rng(B + N)
+    la = -rng.random((B, M, N)).astype(np.float32)
+    lga, lgb = _marginals(B, M, N, rng, rows, cols)
+    P, used, uh, vh = _forward(la, 0.1, T, lga, lgb)
+    assert used == T
+    r, c = np.delete(np.arange(M), rows), np.delete(np.arange(N), cols)
+    # the first iteration starts from v = 0 at every column, so it sees them all
+    lgb1 = lgb[1:2].copy()
+    ref = osk.dual_forward(la[1:2, r], 0.1, T, log_a=lga[1:2, r], log_b=lgb1, keep_history=True)
+    assert not P[1, rows].any() and not P[1][:, cols].any()
+    assert _rel(P[1][np.ix_(r, c)], ref.P[0][:, c]) < TOL
+    scale = max(np.abs(ref.u_hist).max(), np.abs(ref.v_hist[..., c]).max())
+    assert np.abs(uh[:, 1][:, r] - ref.u_hist[:, 0]).max() < TOL * scale
+    assert np.abs(vh[:, 1][:, c] - ref.v_hist[:, 0][:, c]).max() < TOL * scale
+    assert np.isneginf(uh[:, 1][:, rows]).all() and np.isneginf(vh[:, 1][:, cols]).all()
+
+
+@pytest.mark.parametrize("B,M,N", SHAPES)
+def test_zero_marginals_and_the_stop_test(B, M, N):
+    """Rows of zero mass take no part in the stop test after the first iteration."""
+    tol, noise = 1e-5, 5e-7
+    rng = np.random.default_rng(M + 1)
+    la = -rng.random((2, M, N)).astype(np.float32)
+    lga, _ = _marginals(2, M, N, rng, [1, 2, M - 1], [])
+    rep = -(-B // 2)
+    _, used, _, _ = _forward(np.concatenate([la] * rep), 0.2, 50, np.concatenate([lga] * rep), None, tol)
+    r = np.delete(np.arange(M), [1, 2, M - 1])
+    deltas = np.maximum(osk.dual_forward(la[:1], 0.2, 50, log_a=lga[:1]).deltas,
+                        osk.dual_forward(la[1:, r], 0.2, 50, log_a=lga[1:, r]).deltas)
+    assert 1 < used < 50
+    assert deltas[used - 1] < tol + noise and deltas[used - 2] > tol - noise

@@ -203,3 +203,16 @@ def test_tol_below_what_floats_resolve(B, M, N):
     assert 5 < int(counts[0]) <= 40
     ref = osk.dual_forward(la, 0.05, 40)
     assert np.abs(P.cpu().numpy() - ref.P).max() < TOL * ref.P.max()
+
+
+@pytest.mark.parametrize("B,M,N", [(4, 1024, 16384), (16, 1024, 2048), (144, 400, 450)])
+def test_cost_of_long_tiles(B, M, N):
+    """sum(P C) of the returned plan: a lane's entries span e^20, and in one chain
+    over all of them the small ones were lost (-3.3e-7 in the mean).  The fold of
+    the lanes rounds ten times (wave, workgroup, tiles), either way: no more than
+    10 2^-24 for an element, and less than 2^-23 in the mean."""
+    C = torch.rand(B, M, N, generator=torch.Generator(device=DEV).manual_seed(N), device=DEV)
+    res = dot_amd.sinkhorn(C, reg=0.05, n_iters=20, tol=0.0)
+    off = res.cost.double() / (res.transport_plan.double() * C.double()).sum((1, 2)) - 1
+    assert float(off.abs().max()) < 10 * 2.0 ** -24
+    assert abs(float(off.mean())) < 2.0 ** -23

@@ -749,13 +749,13 @@ struct FwdResArgs {
 
 // Bounds of the scaling domain (forward): the column factors V and the row
 // factors w of a workgroup's element stay within them, or the element goes
-// back to the log domain.  An entry E below 2^-126 may be flushed to 0; with
-// M <= 1024 rows its share of a column sum r = sum_i E w is at most
-// 2^10 2^-126 2^40 = 2^-76, and r >= 2^-50 keeps that below 2^-26 of r.  In a
-// row, s >= 2^-40 (the largest E is 1) against 2^10 2^-126 2^40.
+// back to the log domain.  An entry E below 2^-126 may be flushed to 0; the
+// share of M such entries in a column sum r = sum_i E w is at most
+// M 2^-126 2^40, and r >= M 2^-60 keeps that below 2^-26 of r.  In a row of N,
+// s >= 2^-40 (the largest E is 1) against N 2^-126 2^40: 2^-32 at N = 16384.
 constexpr float kScaleMax = 0x1p40f;
 constexpr float kScaleMin = 0x1p-40f;
-constexpr float kScaledColMin = 0x1p-50f;
+__host__ __device__ constexpr float scaled_col_min(int M) { return M > 1024 ? float(M) * 0x1p-60f : 0x1p-50f; }
 
 // E = 2^((x - x_max) kscale log2 e) of a row's scores x, x_max the one whose K is
 // the largest: exactly 1 there, whatever the size of the scores (of a row that
@@ -1043,7 +1043,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
                 part, a.xchg + size_t(cur) * G * a.N, a.N, b, a.W, w, a.tag_base | unsigned(t), local,
                 a.spin_limit, a.status, dead, a.mark, [&](int j, float r) {
                     const float vn = pick(b_own, (j - threadIdx.x) / kThreads) / r;
-                    const bool ok = r >= kScaledColMin && vn >= kScaleMin && vn <= kScaleMax;
+                    const bool ok = r >= scaled_col_min(1024) && vn >= kScaleMin && vn <= kScaleMax;
                     lds_v[cur * a.N + j] = ok ? vn : __builtin_nanf("");
                     low |= !ok;
                 });

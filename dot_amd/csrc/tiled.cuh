@@ -496,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 bool lin = SC, good;
                 if constexpr (SC) {
                     vn = safe_exp(lds_lb[j]) / cs;
-                    good = cs >= res::kScaledColMin && vn >= res::kScaleMin && vn <= res::kScaleMax;
+                    good = cs >= res::scaled_col_min(a.M) && vn >= res::kScaleMin && vn <= res::kScaleMax;
                 } else {
                     good = cs >= sk::kColSumFloor && cs <= FLT_MAX;
                     if (good) vn = lds_lb[j] + lds_v[prev * seg + j] - logf(cs);

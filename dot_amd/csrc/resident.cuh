@@ -1308,6 +1308,10 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     const bool failed = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= a.mark;
     float vf[PL];
     R::load(lds_v + par * a.N, lane, a.N, vf, 0.0f);
+    float vmax = vf[0];
+#pragma unroll
+    for (int e = 1; e < PL; ++e) vmax = fmaxf(vmax, vf[e]);
+    vmax = wave_max(vmax);
     if (a.v_out && w == 0)
         for (int j = threadIdx.x; j < a.N; j += kThreads) {
             const float vj = lds_v[par * a.N + j];
@@ -1334,6 +1338,14 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
                 pv[e] = (x[k][e] * wi) * vf[e];
                 if (a.cost) cacc = fmaf(pv[e], csign * c[e], cacc);
                 if (failed) pv[e] = __builtin_nanf("");
+            }
+            if (wi * vmax > 1.0f) {
+                // an entry whose E was flushed to 0 may be a float's itself: from its score
+                R::load(a.X + (bM + i) * a.N, lane, a.N, c, 0.0f);
+#pragma unroll
+                for (int e = 0; e < PL; ++e)
+                    if (pv[e] == 0.0f && wi * vf[e] > 1.0f)
+                        pv[e] = safe_exp((c[e] * a.kscale + ui) + logf(vf[e]));
             }
             if (a.plan) R::store(a.plan + (bM + i) * a.N, lane, a.N, pv);
             continue;

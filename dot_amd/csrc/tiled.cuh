@@ -806,6 +806,10 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     const bool failed = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
     float vf[PL];
     Rw::load(lds_v + par * seg, lane, nc, vf, 0.0f);
+    float vmax = vf[0];
+#pragma unroll
+    for (int e = 1; e < PL; ++e) vmax = fmaxf(vmax, vf[e]);
+    vmax = wave_max(vmax);
     if (a.v_out && s == 0)
         for (int j = threadIdx.x; j < nc; j += kThreads) {
             const float vj = lds_v[par * seg + j];
@@ -834,6 +838,15 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
             x[e] = failed ? __builtin_nanf("") : p;
         }
         cacc += crow;
+        if (scal && wi * vmax > 1.0f) {
+            // an entry whose E was flushed to 0 may be a float's itself: from its score
+            float xs[PL];
+            load_row(a.X + tile0 + size_t(l) * a.N, xs);
+            const float u = u_of(lds_la[l], q.y, par ? q.w : q.z);
+#pragma unroll
+            for (int e = 0; e < PL; ++e)
+                if (x[e] == 0.0f && wi * vf[e] > 1.0f) x[e] = safe_exp((xs[e] * a.kscale + u) + logf(vf[e]));
+        }
         Rw::store(a.plan + tile0 + size_t(l) * a.N, ln, nc, x);
     };
     const bool scores = a.cost_partial || !scal;

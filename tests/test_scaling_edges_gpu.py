@@ -144,3 +144,19 @@ def test_zero_marginals_and_the_stop_test(B, M, N):
                         osk.dual_forward(la[1:, r], 0.2, 50, log_a=lga[1:, r]).deltas)
     assert 1 < used < 50
     assert deltas[used - 1] < tol + noise and deltas[used - 2] > tol - noise
+
+
+@pytest.mark.parametrize("B,M,N", SHAPES)
+def test_small_plan_entries(B, M, N):
+    """An entry below 2^-126 of its row's kernel, in a column with a large factor,
+    has its own value in the plan (not 0): row 0 sees column 1 2^-131 away, the
+    other rows 2^-33 away."""
+    rng = np.random.default_rng(6)
+    la = -(0.1 * rng.random((B, M, N))).astype(np.float32)
+    la[1, 1:, 1] = -3.3 * np.log(2)
+    la[1, 0, 1] = -9.1
+    P, _, _, vh = _forward(la, 0.1, 12)
+    ref = osk.dual_forward(la[1:2], 0.1, 12)
+    want = ref.P[0, 0, 1]
+    assert 1e-38 < want < 1e-30 and 20 < vh[-1, 1, 1] < 40 * np.log(2)
+    assert abs(P[1, 0, 1] / want - 1) < 1e-4  # exp of a sum of terms of size 91, rounded to 91 2^-24 each

@@ -231,6 +231,66 @@ struct RowGroup {
     }
 };
 
+// Exact max-shifted log-sum-exp of K + u_t (kernels.cu:629-671) over columns of
+// one element: the lanes set in `need` get that of column col0 + lane.  bM is
+// the element's first row; the potentials are awaited under tag t.  The wave's
+// lanes are dealt to the columns (all 64 to one, one to each of 64), each taking
+// four rows at a time, so that a wait covers 4 x 64 rows where a thread per
+// column waited for each row's word.  One far column, 20 iterations at reg 0.01:
+// 3 x 2272 x 80 1316 -> 244 us per call, 4 x 1024 x 16384 2132 -> 1362 (1110
+// without the far column; with the log domain's rows loaded a batch ahead).
+__device__ __forceinline__ float exact_columns(const FwdArgs& a, unsigned long long need, unsigned t, size_t bM,
+                                            int col0, bool& dead) {
+    const int lane = threadIdx.x % kWave;
+    int lg = 6;  // 2^lg lanes per column
+    while ((__popcll(need) << lg) > kWave) --lg;
+    const int sub = lane & ((1 << lg) - 1);
+    unsigned long long left = need;
+    for (int k = lane >> lg; k > 0; --k) left &= left - 1;
+    const bool on = left != 0;
+    const float* col = a.X + bM * a.N + col0 + (on ? __ffsll(left) - 1 : 0);
+    const word_t* urow = a.uslot + size_t(t & 1) * a.B * a.M + bM;
+    constexpr int Q = 4;
+    const int step = 1 << lg;
+    auto terms = [&](int i0, float(&y)[Q]) {  // K + u of this lane's next rows, -inf past the last
+        word_t u[Q];
+        float x[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = min(i0 + q * step, a.M - 1);
+            u[q] = __hip_atomic_load(const_cast<word_t*>(urow + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            x[q] = col[size_t(i) * a.N];
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int i = i0 + q * step;
+            float ui = __uint_as_float(static_cast<unsigned>(u[q]));
+            if (i < a.M && static_cast<unsigned>(u[q] >> 32) != t)
+                ui = res::collect(const_cast<word_t*>(urow + i), t, a.spin_limit, a.status, dead);
+            y[q] = i < a.M ? x[q] * a.kscale + ui : -INFINITY;
+        }
+    };
+    float mx = -FLT_MAX, sm = 0.0f;
+    if (on)
+        for (int i = sub; i < a.M; i += Q * step) {
+            float y[Q];
+            terms(i, y);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) mx = fmaxf(mx, y[q]);
+        }
+    for (int d = step / 2; d > 0; d /= 2) mx = fmaxf(mx, __shfl_xor(mx, d));
+    if (on)
+        for (int i = sub; i < a.M; i += Q * step) {
+            float y[Q];
+            terms(i, y);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) sm += safe_exp(y[q] - mx);
+        }
+    for (int d = step / 2; d > 0; d /= 2) sm += __shfl_xor(sm, d);
+    const float lse = mx + logf(fmaxf(sm, sk::kSumFloor));
+    return __shfl(lse, __popcll(need & ((1ull << lane) - 1)) << lg);
+}
+
 template <int VEC, int CH, int KB, int RR>
 __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     using Rw = Row<VEC, CH>;
@@ -487,40 +547,38 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
             for (int r = 0; r < kColsPerThread; ++r)
                 if (r < mine) red[tid + r * kThreads] = got[r];
             __syncthreads();
-            for (int jj = threadIdx.x; jj < S; jj += kThreads) {
+            for (int first = 0; first < S; first += kThreads) {
+                const int jj = first + int(threadIdx.x);
+                const bool in = jj < S;
                 float cs = 0.0f;
-                for (int g = 0; g < ST; ++g) cs += red[g * S + jj];
+                if (in)
+                    for (int g = 0; g < ST; ++g) cs += red[g * S + jj];
                 if (dead) cs = __builtin_nanf("");
                 const int j = j0 + jj;
+                const float lb = in ? lds_lb[j] : 0.0f;
                 float vn = 0.0f;
                 bool lin = SC, good;
                 if constexpr (SC) {
-                    vn = safe_exp(lds_lb[j]) / cs;
+                    vn = safe_exp(lb) / cs;
                     good = cs >= res::scaled_col_min(a.M) && vn >= res::kScaleMin && vn <= res::kScaleMax;
                 } else {
                     good = cs >= sk::kColSumFloor && cs <= FLT_MAX;
-                    if (good) vn = lds_lb[j] + lds_v[prev * seg + j] - logf(cs);
+                    if (in && good) vn = lb + lds_v[prev * seg + j] - logf(cs);
                 }
                 if (!good) {
-                    // exact max-shifted LSE over the column (kernels.cu:629-671)
-                    const float* col = a.X + bM * a.N + c0 + j;
-                    const word_t* urow = a.uslot + size_t(cur) * a.B * a.M + bM;
-                    float mx = -FLT_MAX;
-                    for (int i = 0; i < a.M; ++i) {
-                        const float ui = res::collect(const_cast<word_t*>(urow + i), tag, a.spin_limit, a.status, dead);
-                        mx = fmaxf(mx, col[size_t(i) * a.N] * a.kscale + ui);
-                    }
-                    float sm = 0.0f;
-                    for (int i = 0; i < a.M; ++i) {
-                        const float ui = __uint_as_float(static_cast<unsigned>(__hip_atomic_load(
-                            const_cast<word_t*>(urow + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
-                        sm += safe_exp(col[size_t(i) * a.N] * a.kscale + ui - mx);
-                    }
-                    vn = lds_lb[j] - (mx + logf(fmaxf(sm, sk::kSumFloor)));
+                    vn = -INFINITY;  // a zero marginal's v, whatever the column (in every iteration: no sum to form)
                     lin = false;
                 }
-                publish(res_row + j, vn, (SC && !lin) ? (tag | kLogBit) : tag, local_col);
-                if (a.v_hist) a.v_hist[(size_t(t - 1) * a.B + b) * a.N + c0 + j] = lin ? logf(vn) : vn;
+                const unsigned long long need = __ballot(in && !good && lb != -INFINITY);
+                // (kept out of the loop's line: in it, 144 x 400 x 450 took 20.3 us per iteration for 18.9)
+                if (__builtin_expect(need != 0, 0)) {
+                    const float x = exact_columns(a, need, tag, bM, c0 + j - lane, dead);
+                    if ((need >> lane) & 1u) vn = lb - x;
+                }
+                if (in) {
+                    publish(res_row + j, vn, (SC && !lin) ? (tag | kLogBit) : tag, local_col);
+                    if (a.v_hist) a.v_hist[(size_t(t - 1) * a.B + b) * a.N + c0 + j] = lin ? logf(vn) : vn;
+                }
             }
         }
         // All of the tile's new factors.
@@ -693,7 +751,11 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
             Rw::load(lds_v + prev * seg, lane, nc, v2, 0.0f);
 #pragma unroll
             for (int e = 0; e < PL; ++e) v2[e] *= kLog2E;
-            auto batch = [&](float(&x)[KB][PL], int k0) {
+            // (the next batch's loads pass under this one's exchange: 16 x 1024 x 2048
+            // 28.5 -> 26.2 us per iteration, 4 x 1024 x 16384 55 -> 51)
+            auto batch = [&](float(&x)[KB][PL], int k0, float(&next)[KB][PL]) {
+                load_rows(a.X, k0 + KB, next);
+                mask_rows(x);
                 float q[KB];
 #pragma unroll
                 for (int r = 0; r < KB; ++r) {
@@ -753,12 +815,11 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
 #pragma unroll
                 for (int e = 0; e < PL; ++e) asm volatile("" : "+v"(acc[e]));  // keep the update here
             };
-            float x[KB][PL];
+            float x[KB][PL], y[KB][PL];
             if (nk > 0) load_rows(a.X, 0, x);
-            for (int k = 0; k < nk; k += KB) {
-                mask_rows(x);
-                batch(x, k);
-                load_rows(a.X, k + KB, x);
+            for (int k = 0; k < nk; k += 2 * KB) {
+                batch(x, k, y);
+                if (k + KB < nk) batch(y, k + KB, x);
             }
             word_t dpre[res::kDeltaPrefetch];
             if (test && wave == 0) prefetch_deltas(t, dpre);
@@ -772,6 +833,14 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
                 break;
             }
         }
+        // (the rows kept in registers are E, which the log domain does not use: their
+        // registers are free for its second buffer)
+#pragma unroll
+        for (int q = 0; q < RR / KB; ++q)
+#pragma unroll
+            for (int r = 0; r < KB; ++r)
+#pragma unroll
+                for (int e = 0; e < PL; ++e) xr[q][r][e] = 0.0f;
     }
     __syncthreads();
     if (leave) {

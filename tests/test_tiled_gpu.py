@@ -216,3 +216,15 @@ def test_cost_of_long_tiles(B, M, N):
     off = res.cost.double() / (res.transport_plan.double() * C.double()).sum((1, 2)) - 1
     assert float(off.abs().max()) < 10 * 2.0 ** -24
     assert abs(float(off.mean())) < 2.0 ** -23
+
+
+@pytest.mark.parametrize("B,M,N", [(2, 333, 1400), (2, 70, 5000), (160, 101, 510), (3, 2272, 80)])
+@pytest.mark.parametrize("far", [1, 2, 3, 17, 0])
+def test_many_columns_leave_at_once(B, M, N, far):
+    """One far column of an element, some, every other one (0): the lanes that
+    form their exact sums are dealt to them."""
+    rng = np.random.default_rng(far + N)
+    la = -(0.1 * rng.random((B, M, N))).astype(np.float32)
+    cols = np.arange(0, N, 2) if far == 0 else rng.choice(N, min(far, N), replace=False)
+    la[1][:, cols] -= 0.7
+    assert _check(la, 0.01, 5, pick=[0, 1]) == 5

@@ -377,10 +377,18 @@ __device__ __forceinline__ void exchange_columns(const float* part, unsigned lon
                                                  int* status, bool& dead, int mark, F&& f) {
     static_assert(NQ >= 1 && NQ <= kColsPerThread, "rows of at most 1024 columns");
     static_assert(MG >= 1 && MG <= kMaxGroup, "at most kMaxGroup workgroups per element");
+    // The addresses and guards below depend only on the thread and the element;
+    // computed from these opaque copies they are rebuilt at each call instead of
+    // being hoisted out of the caller's iteration loop and held in registers for
+    // the whole kernel (C3 adjoint: 70 -> 42 spilled SGPRs, 3 % faster; the
+    // forward's log domain reloaded the fold's addresses from scratch memory one
+    // after the other: 8.4 -> 7.5 us per iteration at 64 x 512 x 512).
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
     float own[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-        const int j = threadIdx.x + q * kThreads;
+        const int j = tid + q * kThreads;
         own[q] = 0.0f;
         if (j < N) {
             float s = 0.0f;
@@ -392,12 +400,6 @@ __device__ __forceinline__ void exchange_columns(const float* part, unsigned lon
     }
     unsigned long long* base = slot + size_t(b) * W * N;
     forced_timeout(spin_limit, status, dead, mark);
-    // The guards below depend only on the thread and the element; computed
-    // from these opaque copies they are rebuilt at each call instead of being
-    // hoisted out of the caller's iteration loop and held in scalar registers
-    // for the whole kernel (C3 adjoint: 70 -> 42 spilled SGPRs, 3 % faster).
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
     asm volatile("" : "+s"(W), "+s"(w));
     // One poll round issues the loads of every (column, workgroup) pair first
     // and only then looks at the tags, so the round costs one memory latency
@@ -909,13 +911,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     float v[PL];  // v_{t-1}, or V_{t-1} in the scaling domain
 #pragma unroll
     for (int e = 0; e < PL; ++e) v[e] = scal ? 1.0f : 0.0f;
-    // log a of the row this lane takes in each group of GR rows
-    float lga_slot[RPW / GR];
-#pragma unroll
-    for (int g = 0; g < RPW / GR; ++g) lga_slot[g] = lds_la[wave + kWaves * (g * GR + slot_of_lane<GR>(lane))];
-    float lse_slot[RPW / GR];  // the same row's log2-sum-exp of the last iteration (the next shift)
-#pragma unroll
-    for (int g = 0; g < RPW / GR; ++g) lse_slot[g] = 0.0f;
     float kscale2 = a.kscale * kLog2E;
     // scheduled runs: this iteration's scale, and the next one's already in flight
     float ks_it = a.kscale;
@@ -1074,7 +1069,117 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
         }
     }
     if (!scal) {
+        auto exact_columns = [&](int t) {
+            const int cur = t & 1;
+            // Exact column LSE of K + u_t over the element's rows: max, then sum.
+            float cm[PL];
+#pragma unroll
+            for (int e = 0; e < PL; ++e) cm[e] = -FLT_MAX;
+#pragma unroll
+            for (int k = 0; k < RPW; ++k) {
+                const int l = wave + kWaves * k;
+                if (row0 + l >= rend) continue;
+                const float u = lds_u[cur * ROWS + l];
+#pragma unroll
+                for (int e = 0; e < PL; ++e)
+                    if (R::valid(lane, e, a.N)) cm[e] = fmaxf(cm[e], fmaf(x[k][e], ks_it, u));
+            }
+            tree_combine<VEC, CH>(cm, part, a.N, OpMax{});
+            unsigned long long* fslot = a.fxchg + size_t(cur) * 2 * G * a.N;
+            if (wave == 0) {
+                unsigned long long* mine = fslot + size_t(gid) * a.N;
+#pragma unroll
+                for (int k = 0; k < CH; ++k)
+#pragma unroll
+                    for (int q = 0; q < VEC; ++q) {
+                        const int col = R::col(lane, k) + q;
+                        if (col < a.N) publish(mine + col, cm[k * VEC + q], a.tag_base | unsigned(t), local);
+                    }
+            }
+            __syncthreads();
+            for (int w2 = wave; w2 < a.W; w2 += kWaves) {
+                float got[PL];
+                collect_row<VEC, CH>(fslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
+                                     a.spin_limit, a.status, dead, got, a.mark);
+                R::store(part + w2 * a.N, lane, a.N, got);
+            }
+            __syncthreads();
+            for (int j = threadIdx.x; j < a.N; j += kThreads) {
+                float mx = -FLT_MAX;
+                for (int w2 = 0; w2 < a.W; ++w2) mx = fmaxf(mx, part[w2 * a.N + j]);
+                lds_mx[j] = mx;
+            }
+            __syncthreads();
+            float mxl[PL], sm[PL];
+            R::load(lds_mx, lane, a.N, mxl, 0.0f);
+#pragma unroll
+            for (int e = 0; e < PL; ++e) sm[e] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < RPW; ++k) {
+                const int l = wave + kWaves * k;
+                if (row0 + l >= rend) continue;
+                const float u = lds_u[cur * ROWS + l];
+#pragma unroll
+                for (int e = 0; e < PL; ++e)
+                    if (R::valid(lane, e, a.N)) sm[e] += safe_exp(fmaf(x[k][e], ks_it, u) - mxl[e]);
+            }
+            tree_combine<VEC, CH>(sm, part, a.N);
+            unsigned long long* sslot = fslot + size_t(G) * a.N;
+            if (wave == 0) {
+                unsigned long long* mine = sslot + size_t(gid) * a.N;
+#pragma unroll
+                for (int k = 0; k < CH; ++k)
+#pragma unroll
+                    for (int q = 0; q < VEC; ++q) {
+                        const int col = R::col(lane, k) + q;
+                        if (col < a.N) publish(mine + col, sm[k * VEC + q], a.tag_base | unsigned(t), local);
+                    }
+            }
+            __syncthreads();
+            for (int w2 = wave; w2 < a.W; w2 += kWaves) {
+                float got[PL];
+                collect_row<VEC, CH>(sslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
+                                     a.spin_limit, a.status, dead, got, a.mark);
+                R::store(part + w2 * a.N, lane, a.N, got);
+            }
+            __syncthreads();
+            for (int j = threadIdx.x; j < a.N; j += kThreads) {
+                const float vj = lds_v[cur * a.N + j];
+                if (vj != vj) {
+                    float s = 0.0f;
+                    for (int w2 = 0; w2 < a.W; ++w2) s += part[w2 * a.N + j];
+                    lds_v[cur * a.N + j] = lds_lb[j] - (lds_mx[j] + logf(fmaxf(s, sk::kSumFloor)));
+                }
+            }
+            __syncthreads();
+        };
+        // v_t to the history and the registers; true once the stop test of iteration t - 1 fired
+        auto finish_iteration = [&](int t) {
+            const int cur = t & 1;
+            if (a.v_hist && w == 0)
+                for (int j = threadIdx.x; j < a.N; j += kThreads)
+                    a.v_hist[(size_t(t - 1) * a.B + b) * a.N + j] = lds_v[cur * a.N + j];
+            if (check && t >= 2 && scratch[0] < a.tol) {
+                used = t - 1;
+                conv = 1;
+                return true;
+            }
+            R::load(lds_v + cur * a.N, lane, a.N, v, 0.0f);
+            return false;
+        };
+        // log a of the row this lane takes in each group of GR rows
+        float lga_slot[RPW / GR];
+#pragma unroll
+        for (int g = 0; g < RPW / GR; ++g) lga_slot[g] = lds_la[wave + kWaves * (g * GR + slot_of_lane<GR>(lane))];
+        float lse_slot[RPW / GR];  // the same row's log2-sum-exp of the last iteration (the next shift)
+#pragma unroll
+        for (int g = 0; g < RPW / GR; ++g) lse_slot[g] = 0.0f;
         bool first = true;  // no LSE of the last iteration to shift by
+        if (resume) {  // (beside the loop, whose registers it would share: 28 spilled instead of 6 for strips of 4 x 16 floats)
+            exact_columns(t0);
+            finish_iteration(t0);
+            ++t0;
+        }
         for (int t = t0; t <= a.max_iter && conv == 0; ++t) {
             const int cur = t & 1, prev = cur ^ 1;
             const bool test = check && t >= 2;
@@ -1084,218 +1189,128 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
                 if (t < a.max_iter) ks_next = a.kscale_t[t];
             }
             unsigned long long dpre[kDeltaPrefetch];
-            if (test && wave == 0 && !resume) prefetch_deltas(t, dpre);
-            int low = resume ? 1 : 0;
-            if (!resume) {
-                // Row update (kernels.cu:503-545) and the shared-exponential column sums,
-                // in base 2: y = K log2(e) + v log2(e), m = max_j y, s = sum_j 2^(y - m),
-                // u = log a - ln2 (m + log2 s), and the column sums take 2^(y - m) a / s.
-                // Rows go in groups of GR: their maxima and sums are reduced across the
-                // wave together (transposed butterfly), and each lane then takes the
-                // logarithm for one row of the group.
-                float acc[PL], v2[PL];
+            if (test && wave == 0) prefetch_deltas(t, dpre);
+            int low = 0;
+            // Row update (kernels.cu:503-545) and the shared-exponential column sums,
+            // in base 2: y = K log2(e) + v log2(e), m = max_j y, s = sum_j 2^(y - m),
+            // u = log a - ln2 (m + log2 s), and the column sums take 2^(y - m) a / s.
+            // Rows go in groups of GR: their maxima and sums are reduced across the
+            // wave together (transposed butterfly), and each lane then takes the
+            // logarithm for one row of the group.
+            float acc[PL], v2[PL];
 #pragma unroll
-                for (int e = 0; e < PL; ++e) {
-                    acc[e] = 0.0f;
-                    v2[e] = v[e] * kLog2E;
-                }
-                float uk[RPW];  // this wave's new u values; stored after the loop, which keeps it branch-free
+            for (int e = 0; e < PL; ++e) {
+                acc[e] = 0.0f;
+                v2[e] = v[e] * kLog2E;
+            }
+            float uk[RPW];  // this wave's new u values; stored after the loop, which keeps it branch-free
 #pragma unroll
-                for (int g0 = 0; g0 < RPW; g0 += GR) {
-                    float y[GR][PL];
-                    // The shift m of a row's exponentials: its log2-sum-exp of the
-                    // previous iteration, which spares the row maximum and keeps the sum
-                    // near 1 once v settles; the row maximum itself in the first
-                    // iteration and whenever the shifted sum leaves [2^-30, 2^30] (a
-                    // large change of v or of the scale, a row without a finite score).
-                    // Within it the largest term is at least 2^-42, so every term that
-                    // matters is a normal float, and the sum is above the floor
-                    // (1e-12) that applies only to a maximum-shifted sum.
-                    auto row_max = [&](const float (&v2)[PL]) {
-                        float lm[GR];
-#pragma unroll
-                        for (int r = 0; r < GR; ++r) {
-                            lm[r] = -FLT_MAX;
-#pragma unroll
-                            for (int e = 0; e < PL; ++e) lm[r] = fmaxf(lm[r], fmaf(x[g0 + r][e], kscale2, v2[e]));
-                        }
-                        return transposed_reduce<GR>(lm, OpMax{});
-                    };
-                    auto shifted_exps = [&](float m, const float (&v2)[PL]) {
-                        float ls[GR];
-#pragma unroll
-                        for (int r = 0; r < GR; ++r) {
-                            const float mr = read_lane(m, lane_of_slot<GR>(r));
-                            ls[r] = 0.0f;
-#pragma unroll
-                            for (int e = 0; e < PL; ++e) {
-                                y[r][e] = __builtin_amdgcn_exp2f(fmaf(x[g0 + r][e], kscale2, v2[e]) - mr);
-                                ls[r] += y[r][e];
-                            }
-                        }
-                        return transposed_sum<GR>(ls);
-                    };
-                    const bool exact = first || !a.lagged_shift;
-                    float m_l = exact ? row_max(v2) : lse_slot[g0 / GR];
-                    float s_sum = shifted_exps(m_l, v2);
-                    if (!exact && !__all(s_sum >= 0x1p-30f && s_sum <= 0x1p30f)) {
-                        // v2 again, opaque to the compiler: kept from sharing the first
-                        // pass's products, whose registers the exponentials then reuse
-                        float v2r[PL];
-#pragma unroll
-                        for (int e = 0; e < PL; ++e) {
-                            v2r[e] = v2[e];
-                            asm volatile("" : "+v"(v2r[e]));
-                        }
-                        m_l = row_max(v2r);
-                        s_sum = shifted_exps(m_l, v2r);
-                    }
-                    const float s_l = fmaxf(s_sum, sk::kSumFloor);
-                    const float lga_l = lga_slot[g0 / GR];
-                    const float lg2 = __builtin_amdgcn_logf(s_l);  // log2
-                    const float lse = m_l + lg2;
-                    lse_slot[g0 / GR] = lse;
-                    const float u_l = lga_l - kLn2 * lse;
-                    const float w_l = __builtin_amdgcn_exp2f(fmaf(lga_l, kLog2E, -lg2));  // a / s
+            for (int g0 = 0; g0 < RPW; g0 += GR) {
+                float y[GR][PL];
+                // The shift m of a row's exponentials: its log2-sum-exp of the
+                // previous iteration, which spares the row maximum and keeps the sum
+                // near 1 once v settles; the row maximum itself in the first
+                // iteration and whenever the shifted sum leaves [2^-30, 2^30] (a
+                // large change of v or of the scale, a row without a finite score).
+                // Within it the largest term is at least 2^-42, so every term that
+                // matters is a normal float, and the sum is above the floor
+                // (1e-12) that applies only to a maximum-shifted sum.
+                auto row_max = [&](const float (&v2)[PL]) {
+                    float lm[GR];
 #pragma unroll
                     for (int r = 0; r < GR; ++r) {
-                        const float wr = read_lane(w_l, lane_of_slot<GR>(r));
-                        uk[g0 + r] = read_lane(u_l, lane_of_slot<GR>(r));
+                        lm[r] = -FLT_MAX;
 #pragma unroll
-                        for (int e = 0; e < PL; ++e) acc[e] = fmaf(y[r][e], wr, acc[e]);
+                        for (int e = 0; e < PL; ++e) lm[r] = fmaxf(lm[r], fmaf(x[g0 + r][e], kscale2, v2[e]));
                     }
-                    // Materialise acc here: left alone, the compiler postpones the updates
-                    // to the end of the loop and keeps every group's exponentials live.
+                    return transposed_reduce<GR>(lm, OpMax{});
+                };
+                auto shifted_exps = [&](float m, const float (&v2)[PL]) {
+                    float ls[GR];
 #pragma unroll
-                    for (int e = 0; e < PL; ++e) asm volatile("" : "+v"(acc[e]));
-                }
-                float dmax = 0.0f;
+                    for (int r = 0; r < GR; ++r) {
+                        const float mr = read_lane(m, lane_of_slot<GR>(r));
+                        ls[r] = 0.0f;
 #pragma unroll
-                for (int k = 0; k < RPW; ++k) {
-                    const int l = wave + kWaves * k;
-                    const int i = row0 + l;
-                    if (i < rend) {
-                        dmax = fmaxf(dmax, fabsf(uk[k] - lds_u[prev * ROWS + l]));
-                        if (lane == 0) {
-                            lds_u[cur * ROWS + l] = uk[k];
-                            if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + i] = uk[k];
+                        for (int e = 0; e < PL; ++e) {
+                            y[r][e] = __builtin_amdgcn_exp2f(fmaf(x[g0 + r][e], kscale2, v2[e]) - mr);
+                            ls[r] += y[r][e];
                         }
                     }
+                    return transposed_sum<GR>(ls);
+                };
+                const bool exact = first || !a.lagged_shift;
+                float m_l = exact ? row_max(v2) : lse_slot[g0 / GR];
+                float s_sum = shifted_exps(m_l, v2);
+                if (!exact && !__all(s_sum >= 0x1p-30f && s_sum <= 0x1p30f)) {
+                    // v2 again, opaque to the compiler: kept from sharing the first
+                    // pass's products, whose registers the exponentials then reuse
+                    float v2r[PL];
+#pragma unroll
+                    for (int e = 0; e < PL; ++e) {
+                        v2r[e] = v2[e];
+                        asm volatile("" : "+v"(v2r[e]));
+                    }
+                    m_l = row_max(v2r);
+                    s_sum = shifted_exps(m_l, v2r);
                 }
-                // The last readers of part (the previous exchange or exact fallback)
-                // are behind the barrier that ends the previous iteration's exchange.
-                R::store(part + wave * a.N, lane, a.N, acc);
-                if (lane == 0) scratch[1 + wave] = dmax;
-                __syncthreads();
-                if (check && threadIdx.x == 0) publish_delta(t);
-                exchange_columns<kColRounds<PL>>(
-                    part, a.xchg + size_t(cur) * G * a.N, a.N, b, a.W, w, a.tag_base | unsigned(t), local, a.spin_limit,
-                    a.status, dead, a.mark,
-                    [&](int j, float cs) {
-                        if (cs >= sk::kColSumFloor && cs <= FLT_MAX) {
-                            lds_v[cur * a.N + j] = lds_lb[j] + lds_v[prev * a.N + j] - logf(cs);
-                        } else {
-                            lds_v[cur * a.N + j] = __builtin_nanf("");  // exact LSE below
-                            low = 1;
-                        }
-                    });
-                if (test && wave == 0) finish_deltas(t, dpre);
-                first = false;
+                const float s_l = fmaxf(s_sum, sk::kSumFloor);
+                const float lga_l = lga_slot[g0 / GR];
+                const float lg2 = __builtin_amdgcn_logf(s_l);  // log2
+                const float lse = m_l + lg2;
+                lse_slot[g0 / GR] = lse;
+                const float u_l = lga_l - kLn2 * lse;
+                const float w_l = __builtin_amdgcn_exp2f(fmaf(lga_l, kLog2E, -lg2));  // a / s
+#pragma unroll
+                for (int r = 0; r < GR; ++r) {
+                    const float wr = read_lane(w_l, lane_of_slot<GR>(r));
+                    uk[g0 + r] = read_lane(u_l, lane_of_slot<GR>(r));
+#pragma unroll
+                    for (int e = 0; e < PL; ++e) acc[e] = fmaf(y[r][e], wr, acc[e]);
+                }
+                // Materialise acc here: left alone, the compiler postpones the updates
+                // to the end of the loop and keeps every group's exponentials live.
+#pragma unroll
+                for (int e = 0; e < PL; ++e) asm volatile("" : "+v"(acc[e]));
             }
-            resume = false;
-            if (__syncthreads_or(low)) {
-                // Exact column LSE of K + u_t over the element's rows: max, then sum.
-                float cm[PL];
+            float dmax = 0.0f;
 #pragma unroll
-                for (int e = 0; e < PL; ++e) cm[e] = -FLT_MAX;
-#pragma unroll
-                for (int k = 0; k < RPW; ++k) {
-                    const int l = wave + kWaves * k;
-                    if (row0 + l >= rend) continue;
-                    const float u = lds_u[cur * ROWS + l];
-#pragma unroll
-                    for (int e = 0; e < PL; ++e)
-                        if (R::valid(lane, e, a.N)) cm[e] = fmaxf(cm[e], fmaf(x[k][e], ks_it, u));
-                }
-                tree_combine<VEC, CH>(cm, part, a.N, OpMax{});
-                unsigned long long* fslot = a.fxchg + size_t(cur) * 2 * G * a.N;
-                if (wave == 0) {
-                    unsigned long long* mine = fslot + size_t(gid) * a.N;
-#pragma unroll
-                    for (int k = 0; k < CH; ++k)
-#pragma unroll
-                        for (int q = 0; q < VEC; ++q) {
-                            const int col = R::col(lane, k) + q;
-                            if (col < a.N) publish(mine + col, cm[k * VEC + q], a.tag_base | unsigned(t), local);
-                        }
-                }
-                __syncthreads();
-                for (int w2 = wave; w2 < a.W; w2 += kWaves) {
-                    float got[PL];
-                    collect_row<VEC, CH>(fslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
-                                         a.spin_limit, a.status, dead, got, a.mark);
-                    R::store(part + w2 * a.N, lane, a.N, got);
-                }
-                __syncthreads();
-                for (int j = threadIdx.x; j < a.N; j += kThreads) {
-                    float mx = -FLT_MAX;
-                    for (int w2 = 0; w2 < a.W; ++w2) mx = fmaxf(mx, part[w2 * a.N + j]);
-                    lds_mx[j] = mx;
-                }
-                __syncthreads();
-                float mxl[PL], sm[PL];
-                R::load(lds_mx, lane, a.N, mxl, 0.0f);
-#pragma unroll
-                for (int e = 0; e < PL; ++e) sm[e] = 0.0f;
-#pragma unroll
-                for (int k = 0; k < RPW; ++k) {
-                    const int l = wave + kWaves * k;
-                    if (row0 + l >= rend) continue;
-                    const float u = lds_u[cur * ROWS + l];
-#pragma unroll
-                    for (int e = 0; e < PL; ++e)
-                        if (R::valid(lane, e, a.N)) sm[e] += safe_exp(fmaf(x[k][e], ks_it, u) - mxl[e]);
-                }
-                tree_combine<VEC, CH>(sm, part, a.N);
-                unsigned long long* sslot = fslot + size_t(G) * a.N;
-                if (wave == 0) {
-                    unsigned long long* mine = sslot + size_t(gid) * a.N;
-#pragma unroll
-                    for (int k = 0; k < CH; ++k)
-#pragma unroll
-                        for (int q = 0; q < VEC; ++q) {
-                            const int col = R::col(lane, k) + q;
-                            if (col < a.N) publish(mine + col, sm[k * VEC + q], a.tag_base | unsigned(t), local);
-                        }
-                }
-                __syncthreads();
-                for (int w2 = wave; w2 < a.W; w2 += kWaves) {
-                    float got[PL];
-                    collect_row<VEC, CH>(sslot + (size_t(b) * a.W + w2) * a.N, a.tag_base | unsigned(t), a.N,
-                                         a.spin_limit, a.status, dead, got, a.mark);
-                    R::store(part + w2 * a.N, lane, a.N, got);
-                }
-                __syncthreads();
-                for (int j = threadIdx.x; j < a.N; j += kThreads) {
-                    const float vj = lds_v[cur * a.N + j];
-                    if (vj != vj) {
-                        float s = 0.0f;
-                        for (int w2 = 0; w2 < a.W; ++w2) s += part[w2 * a.N + j];
-                        lds_v[cur * a.N + j] = lds_lb[j] - (lds_mx[j] + logf(fmaxf(s, sk::kSumFloor)));
+            for (int k = 0; k < RPW; ++k) {
+                const int l = wave + kWaves * k;
+                const int i = row0 + l;
+                if (i < rend) {
+                    dmax = fmaxf(dmax, fabsf(uk[k] - lds_u[prev * ROWS + l]));
+                    if (lane == 0) {
+                        lds_u[cur * ROWS + l] = uk[k];
+                        if (a.u_hist) a.u_hist[(size_t(t - 1) * a.B + b) * a.M + i] = uk[k];
                     }
                 }
-                __syncthreads();
             }
-            if (a.v_hist && w == 0)
-                for (int j = threadIdx.x; j < a.N; j += kThreads)
-                    a.v_hist[(size_t(t - 1) * a.B + b) * a.N + j] = lds_v[cur * a.N + j];
-            if (test && scratch[0] < a.tol) {  // the stop test of iteration t-1 fired
-                used = t - 1;
-                conv = 1;
-                break;
-            }
-            R::load(lds_v + cur * a.N, lane, a.N, v, 0.0f);
+            // The last readers of part (the previous exchange or exact fallback)
+            // are behind the barrier that ends the previous iteration's exchange.
+            R::store(part + wave * a.N, lane, a.N, acc);
+            if (lane == 0) scratch[1 + wave] = dmax;
+            __syncthreads();
+            if (check && threadIdx.x == 0) publish_delta(t);
+            exchange_columns<kColRounds<PL>>(
+                part, a.xchg + size_t(cur) * G * a.N, a.N, b, a.W, w, a.tag_base | unsigned(t), local, a.spin_limit,
+                a.status, dead, a.mark,
+                [&](int j, float cs) {
+                    if (cs >= sk::kColSumFloor && cs <= FLT_MAX) {
+                        lds_v[cur * a.N + j] = lds_lb[j] + lds_v[prev * a.N + j] - logf(cs);
+                    } else if (lds_lb[j] == -INFINITY) {
+                        lds_v[cur * a.N + j] = -INFINITY;  // a zero marginal's, whatever the column
+                    } else {
+                        lds_v[cur * a.N + j] = __builtin_nanf("");  // exact LSE below
+                        low = 1;
+                    }
+                });
+            if (test && wave == 0) finish_deltas(t, dpre);
+            first = false;
+            if (__builtin_expect(__syncthreads_or(low), 0)) exact_columns(t);
+            if (finish_iteration(t)) break;
         }
+        w_l = 0.0f;  // (not read any more: its register is free in the loop)
     }
     if (check && conv == 0 && a.max_iter >= 1) {
         if (global_delta(a, a.max_iter, scratch, dead) < a.tol) conv = 1;  // the last iteration

@@ -30,8 +30,9 @@ The same line carries
   irreducible traffic of its tier — inputs read and output written once (8
   bytes per element in the forward, 12 in the adjoint), plus 4 bytes per
   element-sweep for tiers that re-read the matrix every sweep (the
-  register-resident tier keeps it in VGPRs) — and its arithmetic, 8 flops per
-  element-iteration in the forward and 4 per element-sweep in the adjoint, over
+  register-resident tier keeps it in VGPRs) — and its arithmetic, per
+  element-iteration 4 flops in the forward's scaling domain (resident and tiled
+  tiers) and 8 in its log domain, 4 per element-sweep in the adjoint, over
   the sweeps it executed.  ``hbm`` and ``valu`` give both fractions (8 TB/s,
   157.3 TFLOP/s); ``bound`` names the larger;
 * ``cpu_baseline`` — the reference's own CPU kernels (oracle/_ref, compiled
@@ -294,12 +295,15 @@ def profiled_pass(profiler, names, step, steps, torch):
 # Bytes are the irreducible traffic of the kernel's tier: the register-resident
 # kernels read their inputs and write their output once (the matrix then stays
 # in VGPRs: no bytes per sweep); the persistent and streaming kernels also
-# re-read the matrix every sweep.  Forward: read C, write P (8); adjoint: read
-# P and C, write the gradient (12).  Flops per sweep: the forward's row update
-# and shared-exponential column sum (FMA, max, subtract, exp2, add, FMA, plus
-# the column FMA: 8), the adjoint's row dot and column sum (two FMAs: 4).
+# re-read the matrix every sweep.  Forward: read C, write P (8), on the tiles
+# also E written and C read again (16); adjoint: read P and C, write the
+# gradient (12).  Flops per sweep: two FMAs (4) in the forward's scaling domain
+# (resident, tiled) and in the adjoint's row dot and column sum; the forward's
+# log-domain row update and shared-exponential column sum (FMA, max, subtract,
+# exp2, add, FMA, plus the column FMA: 8) in the other tiers.
 KERNEL_WORK = {
-    "sk_fwd_resident": (8.0, 0.0, 8.0, "T_f"),
+    "sk_fwd_resident": (8.0, 0.0, 4.0, "T_f"),
+    "sk_fwd_tiled": (16.0, 4.0, 4.0, "T_f"),
     "sk_imp_resident": (12.0, 0.0, 4.0, "T_b"),
     "sk_fwd_persistent": (8.0, 4.0, 8.0, "T_f"),
     "sk_imp_persistent": (12.0, 4.0, 4.0, "T_b"),
@@ -327,6 +331,7 @@ def sinkhorn_roofline(dominant, stats, E, T_f, T_b, workload):
         "GBps": round(traffic / avg_s / 1e9, 1), "frac": round(traffic / avg_s / 1e9 / HBM_PEAK_GBPS, 4)}
     tier = ("register-resident (one launch, the matrix held in VGPRs for every sweep)" if "resident" in dominant
             else "persistent streaming (one launch; the matrix is re-read every sweep)" if "persistent" in dominant
+            else "tiled persistent (one launch; the scaled kernel is re-read every sweep)" if "tiled" in dominant
             else "streaming sweeps (one launch per sweep)")
     common = {"kernel": dominant, "tier": tier, "sweeps_per_launch": sweeps, "avg_us": round(avg_s * 1e6, 2),
               "bytes_per_launch": bytes_launch, "bytes_per_elem": {"once": once, "per_sweep": per_sweep},
@@ -343,7 +348,7 @@ def sinkhorn_roofline(dominant, stats, E, T_f, T_b, workload):
 
 
 SINKHORN_KERNELS = ["sk_fwd_sweep", "sk_imp_sweep", "sk_fwd_resident", "sk_imp_resident",
-                    "sk_fwd_persistent", "sk_imp_persistent", "mth_sweep", "mth_vfinish",
+                    "sk_fwd_persistent", "sk_imp_persistent", "sk_fwd_tiled", "mth_sweep", "mth_vfinish",
                     "sk_fwd_wide_rows", "sk_fwd_wide_cols", "sk_imp_wide_rows", "sk_imp_wide_cols",
                     "sk_unr_step", "sk_unr_init", "sk_unr_fold", "sk_unr_resident", "sk_unr_persistent"]
 

@@ -5,9 +5,15 @@
  * owned by the caller (fp32 unless stated); the library allocates nothing on
  * its hot path: scratch comes from the caller's `workspace`, sized by the
  * matching *_workspace_bytes() query.  All work is enqueued on `stream`
- * (a hipStream_t); no call synchronises the device.  Functions return
- * DOT_OK (0) or a DOT_ERR_* code; dot_last_error() gives the message for the
- * calling thread.
+ * (a hipStream_t).  Three calls may wait on their stream from the host, none
+ * of them while it is being captured: dot_sinkhorn_forward_method every 16
+ * iterations and dot_sinkhorn_forward on shapes of one launch pair per
+ * iteration (batches beyond the chip) after iterations 4, 8, 16, ..., both
+ * with tol > 0 only; and dot_sinkhorn_backward_implicit on rows of more than
+ * 4096 columns after sweeps 4, 6, ..., 16, 32, 64, ..., whatever tol the
+ * forward had, unless DOT_SK_EXACT_SWEEPS is set.  No other call synchronises.
+ * Functions return DOT_OK (0) or a DOT_ERR_* code; dot_last_error() gives the
+ * message for the calling thread.
  *
  * Layouts: matrices are row-major [B, M, N] (B batch elements, M rows, N
  * columns); row vectors are [B, M]; column vectors are [B, N].
@@ -58,7 +64,8 @@ typedef struct {
     float tol;             /* > 0: stop after the first iteration with max|u_t - u_{t-1}| < tol
                               over the whole batch; <= 0: run max_iter iterations */
     int flags;             /* DOT_SK_* */
-    float* plan;           /* [B,M,N] out: P (or log P); may be NULL */
+    float* plan;           /* [B,M,N] out: P (or log P); may be NULL; the call may use it as
+                              scratch before it holds the result */
     float* cost;           /* [B] out: sum(P * C) with C = -log_alpha; may be NULL */
     float* u_out;          /* [B,M] out: final row potential; may be NULL */
     float* v_out;          /* [B,N] out: final column potential; may be NULL */
@@ -222,10 +229,13 @@ typedef struct {
  * lambda_i = (sum_k P G - sum_k P mu_k) / max(sum_k P, 1e-12),
  * mu_k = (sum_i P G - sum_i P lambda_i) / max(sum_i P, 1e-12),
  * grad = P (G - lambda_i - mu_k) / tau, grad_tau = -sum(grad * log_alpha) / tau.
- * Without DOT_SK_EXACT_SWEEPS, rows of at most 4096 columns (the register-
- * resident and persistent tiers, batches beyond the chip in slabs of them)
- * end a batch element's sweeps early once
- * they have converged, with d = max|mu_t - mu_{t-1}| and s the size of the
+ * Without DOT_SK_EXACT_SWEEPS a batch element's sweeps end early once
+ * they have converged (in one launch on rows of at most 4096 columns: the
+ * register-resident and persistent tiers, batches beyond the chip in slabs of
+ * them; on longer rows, which take launches per sweep, the call also waits on
+ * the stream after sweeps 4, 6, ..., 16, 32, 64, ... below `iters` for the
+ * count of elements left, and launches no more once it is 0; under capture it
+ * records every launch, and those of converged elements return at once), with d = max|mu_t - mu_{t-1}| and s the size of the
  * mu update's operands, max_k (|sum_i P G| + |sum_i P lambda|) / sum_i P:
  * when a sweep leaves mu unchanged (a fixed point: the result is the full
  * count's bit for bit); when three successive changes each shrank by at least
@@ -234,8 +244,9 @@ typedef struct {
  * excludes for a nonzero change (the sweeps have reached their fp32 rounding
  * floor), while at most 2^-18 s.  The
  * reference's GPU op runs every sweep (kernels.cu:1715-1718); its CPU op also
- * stops early, at a change below 1e-6 (kernels_cpu.cpp:276-312).  Other shapes
- * run every sweep.  sweeps_used reports what ran.
+ * stops early, at a change below 1e-6 (kernels_cpu.cpp:276-312).  Shapes of at
+ * most 4096 columns that fit neither tier run every sweep.  sweeps_used reports
+ * what ran.
  * Replaces sinkhorn_backward_implicit_cuda (src/sinkhorn/kernels.cuh:325;
  * kernels.cu:1682-1726) behind sinkhorn_with_grads_implicit
  * (torch_cuda.cpp:803-871; registry.cpp:56). */

@@ -86,15 +86,20 @@ def test_masked_by_a_sum(B, M, N, far):
 
 
 @pytest.mark.parametrize("B,M,N", SHAPES)
-def test_scores_beyond_the_range_of_k(B, M, N):
-    """A score whose K overflows to +inf has no plan; the other elements are not touched by it."""
+@pytest.mark.parametrize("score", [1e38, np.inf, np.nan])
+def test_scores_beyond_the_range_of_k(B, M, N, score):
+    """A score whose K is +inf or NaN: the other elements are not touched by it,
+    and the potentials of its element stay free of NaN (one whose K overflows, or
+    is infinite, has u = -inf)."""
     rng = np.random.default_rng(N)
     la = -rng.random((B, M, N)).astype(np.float32)
-    la[1, 3, 7] = 1e38
-    P, used, _, _ = _forward(la, 0.1, 3)
+    la[1, 3, 7] = score
+    P, used, uh, vh = _forward(la, 0.1, 3)
     assert used == 3
     ref = osk.dual_forward(la[:1], 0.1, 3)
     assert _rel(P[:1], ref.P) < TOL
+    assert not np.isnan(uh[:, 1]).any() and not np.isnan(vh[:, 1]).any()
+    assert np.isneginf(uh[:, 1, 3]).all() == (not np.isnan(score))
 
 
 def _marginals(B, M, N, rng, zero_rows, zero_cols):

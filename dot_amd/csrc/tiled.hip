@@ -104,6 +104,12 @@ bool launch_tiled_forward(til::FwdArgs& a, const TiledCfg& c, bool vec4, bool co
         ProfScope prof("sk_fwd_tiled", stream);
         ok = launch_persistent(kernel, a, grid, res::kThreads, lds, stream);
     };
+    // Batches of KB rows and RR rows kept in registers, us per iteration (RR = RR / 2,
+    // 0, 1.5 RR; then KB / 2, 2 KB at the same RR): 16 x 1024 x 2048 17.6 (19.3, 21.1,
+    // 24.8; 23.0, 52.7), 4 x 4096 x 4096 39.5 (41.4, 42.2, 47.8; 50.7, 78), 4 x 1024 x
+    // 16384 39.6 (40.9, 43.4, 55; 47.0, 79).  Scalar rows: KB / 2 and 2 KB are slower as
+    // well; RR = 8 and 4 are faster at rows of 2047 (18.1 for 19.7) and 16381 (40.7 for
+    // 44.4) and equal at 450 and 1001.
     if (vec4) {
         if (c.narrow) launch(til::forward<4, 2, 4, 8>);
         else launch(til::forward<4, 4, 2, 4>);

@@ -102,8 +102,10 @@ struct FwdSweepArgs {
 //   v_j' = log b_j - LSE_i(K_ij + u_i) = log b_j + v_j - log colsum_j.
 // The row is reduced in base 2 (y = K log2 e + v log2 e, m = max y,
 // s = sum 2^(y - m), u = log a - ln2 (m + log2 s)), the same arithmetic as
-// the register-resident and persistent forwards, so that every tier rounds
-// u alike and the stop test fires at the same iteration on every tier.
+// the register-resident and persistent forwards' log domain, so that these
+// tiers round u alike and their stop test fires at the same iteration.  (In the
+// scaling domain it sees ratios of row sums instead and also fires where the
+// rounding of u, 2^-24 |u|, stays above tol.)
 template <int VEC, int CH>
 __global__ __launch_bounds__(kBlock) void fwd_sweep(FwdSweepArgs a) {
     if (stopped_before(a.delta_bits, a.t, a.tol)) return;

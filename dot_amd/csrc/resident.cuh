@@ -1330,10 +1330,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
     const bool failed = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= a.mark;
     float vf[PL];
     R::load(lds_v + par * a.N, lane, a.N, vf, 0.0f);
-    float vmax = vf[0];
-#pragma unroll
-    for (int e = 1; e < PL; ++e) vmax = fmaxf(vmax, vf[e]);
-    vmax = wave_max(vmax);
     if (a.v_out && w == 0)
         for (int j = threadIdx.x; j < a.N; j += kThreads) {
             const float vj = lds_v[par * a.N + j];
@@ -1361,14 +1357,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
                 if (a.cost) cacc = fmaf(pv[e], csign * c[e], cacc);
                 if (failed) pv[e] = __builtin_nanf("");
             }
-            if (wi * vmax > 1.0f) {
-                // an entry whose E was flushed to 0 may be a float's itself: from its score
-                R::load(a.X + (bM + i) * a.N, lane, a.N, c, 0.0f);
-#pragma unroll
-                for (int e = 0; e < PL; ++e)
-                    if (pv[e] == 0.0f && wi * vf[e] > 1.0f)
-                        pv[e] = safe_exp((c[e] * a.kscale + ui) + logf(vf[e]));
-            }
             if (a.plan) R::store(a.plan + (bM + i) * a.N, lane, a.N, pv);
             continue;
         }
@@ -1380,6 +1368,32 @@ __global__ __launch_bounds__(kThreads) void forward(FwdResArgs a) {
             if (failed) pv[e] = __builtin_nanf("");
         }
         if (a.plan) R::store(a.plan + (bM + i) * a.N, lane, a.N, pv);
+    }
+    if (scal && a.plan && !failed) {
+        // An entry whose E was flushed to 0 may be a float's itself where w V passes 1:
+        // formed from its score, in a pass of its own over such rows.
+        float vmax = vf[0];
+#pragma unroll
+        for (int e = 1; e < PL; ++e) vmax = fmaxf(vmax, vf[e]);
+        vmax = wave_max(vmax);
+        if (__any(row_ok && w_l * vmax > 1.0f)) {
+#pragma unroll
+            for (int k = 0; k < RPW; ++k) {
+                const int l = wave + kWaves * k;
+                const int i = row0f + l;
+                const float wi = read_lane(w_l, lane_of_slot<RPW>(k));
+                if (i >= rend || !(wi * vmax > 1.0f)) continue;
+                const float ui = lds_u[par * ROWS + l];
+                float c[PL], pv[PL];
+                R::load(a.X + (bM + i) * a.N, lane, a.N, c, 0.0f);
+#pragma unroll
+                for (int e = 0; e < PL; ++e) {
+                    pv[e] = (x[k][e] * wi) * vf[e];
+                    if (pv[e] == 0.0f && wi * vf[e] > 1.0f) pv[e] = safe_exp((c[e] * a.kscale + ui) + logf(vf[e]));
+                }
+                R::store(a.plan + (bM + i) * a.N, lane, a.N, pv);
+            }
+        }
     }
     if (a.cost) {
         const float cs = block_reduce<kWaves>(wave_sum(cacc), scratch + 16, OpSum{});

@@ -875,10 +875,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
     const bool failed = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
     float vf[PL];
     Rw::load(lds_v + par * seg, lane, nc, vf, 0.0f);
-    float vmax = vf[0];
-#pragma unroll
-    for (int e = 1; e < PL; ++e) vmax = fmaxf(vmax, vf[e]);
-    vmax = wave_max(vmax);
     if (a.v_out && s == 0)
         for (int j = threadIdx.x; j < nc; j += kThreads) {
             const float vj = lds_v[par * seg + j];
@@ -907,15 +903,6 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
             x[e] = failed ? __builtin_nanf("") : p;
         }
         cacc += crow;
-        if (scal && wi * vmax > 1.0f) {
-            // an entry whose E was flushed to 0 may be a float's itself: from its score
-            float xs[PL];
-            load_row(a.X + tile0 + size_t(l) * a.N, xs);
-            const float u = u_of(lds_la[l], q.y, par ? q.w : q.z);
-#pragma unroll
-            for (int e = 0; e < PL; ++e)
-                if (x[e] == 0.0f && wi * vf[e] > 1.0f) x[e] = safe_exp((xs[e] * a.kscale + u) + logf(vf[e]));
-        }
         Rw::store(a.plan + tile0 + size_t(l) * a.N, ln, nc, x);
     };
     const bool scores = a.cost_partial || !scal;
@@ -933,6 +920,31 @@ __global__ __launch_bounds__(kThreads) void forward(FwdArgs a) {
 #pragma unroll
         for (int r = 0; r < KB; ++r)
             if (k + r < nk) write_row(wave + kWaves * (k + r), x[r], x[r], scores, pst::opaque_lane());
+    }
+    if (scal) {
+        // An entry whose E was flushed to 0 may be a float's itself where w V passes 1:
+        // formed from its score, in a pass of its own over such rows (inside the one
+        // above, its branch cost every call 5 of 147 us at 16 x 1024 x 2048).
+        float vmax = vf[0];
+#pragma unroll
+        for (int e = 1; e < PL; ++e) vmax = fmaxf(vmax, vf[e]);
+        vmax = wave_max(vmax);
+        bool any = false;
+        for (int k = lane; k < nk; k += kWave) any = any || lds_row4[wave + kWaves * k].x * vmax > 1.0f;
+        for (int k = 0; __any(any) && k < nk; ++k) {
+            const int l = wave + kWaves * k;
+            const float4 q = lds_row4[l];
+            if (!(q.x * vmax > 1.0f)) continue;
+            const size_t at = tile0 + size_t(l) * a.N;
+            float p[PL], sc[PL];
+            load_row(a.plan + at, p);
+            load_row(a.X + at, sc);
+            const float u = u_of(lds_la[l], q.y, par ? q.w : q.z);
+#pragma unroll
+            for (int e = 0; e < PL; ++e)
+                if (p[e] == 0.0f && q.x * vf[e] > 1.0f) p[e] = safe_exp((sc[e] * a.kscale + u) + logf(vf[e]));
+            Rw::store(a.plan + at, lane, nc, p);
+        }
     }
     if (a.cost_partial) {
         const float cs = block_reduce<kWaves>(wave_sum(cacc), scratch + 16, OpSum{});
